@@ -18,6 +18,7 @@
 // These are latency-bound per token (a few KB each); only the GEMVs stream
 // HBM.
 #include "common.h"
+#include "mfma_pipe.h"
 
 namespace reng {
 
@@ -364,8 +365,8 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_split(
     }
 }
 
-// attention_split for head_dim % 8 == 0, head_dim <= 128 and 16-byte aligned
-// q, caches: a lane holds eight dimensions (one 16-byte piece) of a key row
+// attention_split for head_dim % 8 == 0, head_dim <= 128 (64 and 128 take
+// attention_stream) and 16-byte aligned q, caches: a lane holds eight dimensions (one 16-byte piece) of a key row
 // and of the same value row, 16 lanes a row, so phase 2 accumulates the rows
 // phase 1 scored, from registers, eight dimensions per lane; the lanes of one
 // piece are summed across the wave (xor 16, 32) and across the waves in LDS.
@@ -505,6 +506,282 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_split16(
         float *ml = part + (size_t)gridDim.x * nh * hd;
         ml[((size_t)s * nh + h0 + tid) * 2] = mrun[tid];
         ml[((size_t)s * nh + h0 + tid) * 2 + 1] = lrun[tid];
+    }
+}
+
+// attention_stream: the same product for head_dim 64 or 128 and 16-byte
+// aligned q and caches. It streams the cache and is bound by HBM (or, in one
+// pass, by the 64 bytes a clock one CU takes in); nothing else should show.
+//
+// A wave works alone on tiles of 64 rows, all of a tile's keys (to the wave's
+// own LDS) and values (to registers) requested at once, 32 KB a wave at
+// head_dim 128; the next tile's keys as soon as the scores have used up this
+// one's, its values behind the accumulation. There is no barrier inside the
+// loop, so no wave waits for another's loads. Scores come from the matrix
+// cores: A is q with head (m & 3) in row m, B sixteen key rows, so every
+// 16-lane group of D holds all four heads' scores of the sixteen keys, and
+// taking D of block g in lane group g leaves lane l with key l. Probabilities
+// stay f32: the values are accumulated by f32 multiply-adds, each lane HD / 16
+// dimensions of rows 16 g .. 16 g + 15 in lane group g, p broadcast inside the
+// group by DPP. The running maximum is the lane group's own, so the loop
+// reduces over 16 lanes only; groups and waves meet once at the end. Loads are
+// bounds-checked buffer loads: value rows past the end read as zeros, and
+// scores past it are replaced by -infinity whatever the keys were.
+//
+// The keys go through LDS for the sake of the request pattern: a B operand
+// loaded straight from the cache takes 64 bytes of each of sixteen rows per
+// instruction, and half-used lines let one CU take in about 16 bytes a clock
+// where whole rows let it take 54. Chunk c of a row lies in slot c ^ f(row),
+// f chosen so that the sixteen rows of an operand read use distinct banks.
+//
+// Up to GB query heads of one key/value head are served by a wave, and hgw
+// waves side by side take the same rows for as many groups of heads, so that
+// the rows come from HBM once and from L2 after that.
+//
+// One call, 32 heads on 8 of 128 dimensions, attention_split16 before: 64 rows
+// 5.9 -> 4.0 us, 512 rows 8.6 -> 6.0, 4096 rows 14.8 -> 12.0, 32768 rows 47.3
+// -> 31.8 (the rows at 4.9 TB/s, then the merge); 28 heads on 4, 32768 rows:
+// 88.8 -> 24.2; 40 on 8: 121 -> 38.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int ATS_TILE = 64, ATS_WAVES = 8, ATS_ONE_PASS_MAX = 1024;
+
+template <int CTRL>
+__device__ __forceinline__ float row16_max_step(float v) {
+    return fmaxf(v, dpp_mov<CTRL, 0xf>(v));
+}
+// Max and sum over each 16-lane row, in every lane of it (row_ror 8, 4, 2, 1).
+__device__ __forceinline__ float row16_max_all(float v) {
+    return row16_max_step<0x121>(row16_max_step<0x122>(row16_max_step<0x124>(row16_max_step<0x128>(v))));
+}
+__device__ __forceinline__ float row16_sum_all(float v) {
+    v += dpp_mov<0x128, 0xf>(v);
+    v += dpp_mov<0x124, 0xf>(v);
+    v += dpp_mov<0x122, 0xf>(v);
+    v += dpp_mov<0x121, 0xf>(v);
+    return v;
+}
+
+// exp(v - m), and 0 where m is -infinity: nothing but -infinity scores so far.
+__device__ __forceinline__ float exp_from(float v, float m) { return m == -INFINITY ? 0.0f : expf(v - m); }
+
+// 16 bytes per lane from r at off into LDS at l + 16 * lane (l wave-uniform).
+__device__ __forceinline__ void buf_copy16_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t off, uint8_t *l) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)l, 16, (int)off, 0, 0, 0);
+}
+
+template <int DPL>
+struct Values;
+template <>
+struct Values<8> {
+    u32x4 w;
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+        w = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+    }
+};
+template <>
+struct Values<4> {
+    u32x2 w;
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+        w = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
+    }
+};
+
+// Rows I .. 15 of each lane group: o += p v.
+template <int I, int GB, int DPL>
+__device__ __forceinline__ void accumulate_rows(const float (&p)[4], const Values<DPL> (&v)[16],
+                                                float (&o)[GB][DPL]) {
+    if constexpr (I < 16) {
+        float x[DPL];
+#pragma unroll
+        for (int e = 0; e < DPL / 2; ++e) {
+            x[2 * e] = __uint_as_float(v[I].w[e] << 16);
+            x[2 * e + 1] = __uint_as_float(v[I].w[e] & 0xffff0000u);
+        }
+#pragma unroll
+        for (int h = 0; h < GB; ++h) {
+            const float pb = dpp_mov<0x150 + I, 0xf>(p[h]);   // row_newbcast:I
+#pragma unroll
+            for (int e = 0; e < DPL; ++e) o[h][e] = fmaf(pb, x[e], o[h][e]);
+        }
+        accumulate_rows<I + 1, GB, DPL>(p, v, o);
+    }
+}
+
+template <int HD, int GB>
+__global__ __launch_bounds__(64 * ATS_WAVES) void attention_stream(
+    const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc, uint32_t nh,
+    uint32_t nkv, uint32_t len, uint32_t chunk, uint32_t hgw, float scale, float *__restrict__ part,
+    uint16_t *__restrict__ out) {
+    constexpr int STEPS = HD / 32, DPL = HD / 16, N = GB * DPL;
+    constexpr int CH = HD / 8, STAGE = ATS_TILE * HD * 2;   // 16-byte chunks of a row; bytes of a tile's keys
+    extern __shared__ __attribute__((aligned(16))) uint8_t stage[];   // [waves][STAGE], then each wave's o
+    __shared__ float mw[ATS_WAVES][GB], lw[ATS_WAVES][GB];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t slots = (blockDim.x >> 6) / hgw;   // tiles side by side
+    const uint32_t s = blockIdx.x, per_kv = nh / nkv;
+    // y walks the key/value heads fastest: the groups of one sit gridDim.x *
+    // nkv workgroups apart, on one XCD when that is a multiple of 8, and share
+    // its rows in L2.
+    const uint32_t g = blockIdx.y % nkv, hb = blockIdx.y / nkv * hgw * GB;   // the workgroup's first head of g
+    const uint32_t hg = hb + wave % hgw * GB;                                // the wave's
+    const uint32_t hn = hg < per_kv ? min((uint32_t)GB, per_kv - hg) : 0;
+    const uint32_t pitch = nkv * HD * 2;   // bytes
+    const uint32_t j0 = s * chunk, j1 = min(len, j0 + chunk);
+
+    bf16x8_t qv[STEPS];
+    const uint16_t *qh = q + (size_t)(g * per_kv + (hn ? hg + min(l16 & 3, hn - 1) : 0)) * HD + 8 * lg;
+#pragma unroll
+    for (int st = 0; st < STEPS; ++st) qv[st] = *reinterpret_cast<const bf16x8_t *>(qh + 32 * st);
+
+    uint8_t *ks = stage + wave * STAGE;
+    Values<DPL> vf[16];
+    // The tile's rows as a buffer that ends with the last row's head.
+    auto rsrc = [&](const uint16_t *base, uint32_t t0) {
+        const uint32_t n = min((uint32_t)ATS_TILE, j1 - t0);
+        const uint8_t *b = reinterpret_cast<const uint8_t *>(base) + (size_t)t0 * pitch + g * (HD * 2);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(b), 0, (int)((n - 1) * pitch + HD * 2),
+                                                 0x00027000);
+    };
+    auto slot = [](uint32_t row, uint32_t c) { return c ^ (CH == 16 ? row & 15 : (row >> 1) & 7); };
+    auto load_keys = [&](uint32_t t0) {
+        const auto r = rsrc(kc, t0);
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const uint32_t row = i * (64 / CH) + lane / CH;
+            buf_copy16_to_lds(r, row * pitch + 16 * slot(row, lane % CH), ks + 1024 * i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load_values = [&](uint32_t t0) {
+        const auto r = rsrc(vc, t0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) vf[i].load(r, (16 * lg + i) * pitch + l16 * (DPL * 2));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float m[GB], l[GB], o[GB][DPL];
+#pragma unroll
+    for (int h = 0; h < GB; ++h) {
+        m[h] = -INFINITY;
+        l[h] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < DPL; ++e) o[h][e] = 0.0f;
+    }
+    float p[4];
+    auto scores = [&](uint32_t t0) {
+        // The keys have landed; the 16 value loads asked for after them may be under way.
+        pipe::wait_vmcnt<16>();
+        asm volatile("" ::: "memory");
+        f32x4 d[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            d[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int st = 0; st < STEPS; ++st) {
+                const uint32_t row = 16 * b + l16;
+                const auto kf = *reinterpret_cast<const bf16x8_t *>(ks + row * (HD * 2) + 16 * slot(row, 4 * st + lg));
+                d[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qv[st], kf, d[b], 0, 0, 0);
+            }
+        }
+        pipe::wait_lgkm0();   // before the next tile's keys overwrite these
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < GB; ++h) {
+            const float lo = lg & 1 ? d[1][h] : d[0][h], hi = lg & 1 ? d[3][h] : d[2][h];
+            p[h] = t0 + lane < j1 ? (lg & 2 ? hi : lo) * scale : -INFINITY;
+        }
+    };
+    auto softmax = [&]() {
+#pragma unroll
+        for (int h = 0; h < GB; ++h) {
+            const float mo = m[h], mn = fmaxf(mo, row16_max_all(p[h]));
+            const float c = exp_from(mo, mn);
+            p[h] = exp_from(p[h], mn);
+            m[h] = mn;
+            l[h] = l[h] * c + p[h];
+#pragma unroll
+            for (int e = 0; e < DPL; ++e) o[h][e] *= c;
+        }
+    };
+    uint32_t t0 = j0 + wave / hgw * ATS_TILE;
+    if (hn && t0 < j1) {
+        const uint32_t step = slots * ATS_TILE;
+        load_keys(t0);
+        load_values(t0);
+        for (; t0 + step < j1; t0 += step) {
+            scores(t0);
+            load_keys(t0 + step);
+            softmax();
+            __builtin_amdgcn_sched_barrier(0);   // values unpacked early would spill
+            accumulate_rows<0, GB, DPL>(p, vf, o);
+            load_values(t0 + step);
+        }
+        scores(t0);
+        softmax();
+        __builtin_amdgcn_sched_barrier(0);
+        accumulate_rows<0, GB, DPL>(p, vf, o);
+    }
+
+    // The lane groups of a wave: to the wave's maximum, then summed. Each swap
+    // exchanges half the lanes of two registers, so the sum of the pair holds
+    // one value in the low half (even rows) and the other in the high half.
+#pragma unroll
+    for (int h = 0; h < GB; ++h) {
+        float M = fmaxf(m[h], __shfl_xor(m[h], 16, 64));
+        M = fmaxf(M, __shfl_xor(M, 32, 64));
+        const float f = exp_from(m[h], M);
+        float ls = row16_sum_all(l[h] * f);
+        ls += __shfl_xor(ls, 16, 64);
+        ls += __shfl_xor(ls, 32, 64);
+#pragma unroll
+        for (int e = 0; e < DPL; ++e) o[h][e] *= f;
+        if (lane == 0) {
+            mw[wave][h] = M;
+            lw[wave][h] = ls;
+        }
+    }
+    float *op = reinterpret_cast<float *>(ks);   // [GB][HD]; the keys are done with
+    float r[N / 2];
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+        const int k = i + N / 2;
+        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[i / DPL][i % DPL]),
+                                                        __float_as_uint(o[k / DPL][k % DPL]), false, false);
+        r[i] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) {
+        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(r[i]), __float_as_uint(r[i + N / 4]), false,
+                                                        false);
+        const uint32_t k = lg * (N / 4) + i;   // this lane group's value
+        op[k / DPL * HD + l16 * DPL + k % DPL] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+    }
+    __syncthreads();
+    // The waves.
+    const uint32_t heads = min(hgw * GB, per_kv - hb), h0 = g * per_kv + hb;
+    for (uint32_t i = tid; i < heads * HD; i += blockDim.x) {
+        const uint32_t h = i / HD % GB, w0 = i / HD / GB;
+        float M = mw[w0][h];
+        for (uint32_t k = 1; k < slots; ++k) M = fmaxf(M, mw[w0 + k * hgw][h]);
+        float v = 0.0f, ls = 0.0f;
+        for (uint32_t k = 0; k < slots; ++k) {
+            const uint32_t w = w0 + k * hgw;
+            const float f = exp_from(mw[w][h], M);
+            v += f * reinterpret_cast<const float *>(stage + w * STAGE)[h * HD + i % HD];
+            ls += f * lw[w][h];
+        }
+        if (part == nullptr) {
+            out[(size_t)h0 * HD + i] = f32_bf16(v / ls);
+        } else {
+            part[((size_t)s * nh + h0) * HD + i] = v;
+            if (i % HD == 0) {
+                float *ml = part + (size_t)gridDim.x * nh * HD;
+                ml[((size_t)s * nh + h0 + i / HD) * 2] = M;
+                ml[((size_t)s * nh + h0 + i / HD) * 2 + 1] = ls;
+            }
+        }
     }
 }
 
@@ -669,9 +946,62 @@ int attention_args(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v
     return RENG_HIP_OK;
 }
 
+// Whole tiles per split, so that no wave runs a part-filled one but the last:
+// never more splits than attn_plan's, whose workspace they use. One pass up to
+// 1024 rows, where the merge's launch costs more than the split saves (one
+// pass / split, 32 heads on 8 of 128 dimensions: 7.1 / 9.1 us at 768 rows, 9.0
+// / 9.7 at 1024, 25 / 12 at 4096; 8 heads on 2 of 64: 6.5 / 8.2 at 1024).
+AttnPlan stream_plan(AttnPlan p, size_t len) {
+    if (p.splits < 2 || len <= (size_t)ATS_ONE_PASS_MAX) return {1u, (uint32_t)len};
+    p.chunk = (p.chunk + ATS_TILE - 1) / ATS_TILE * ATS_TILE;
+    p.splits = (uint32_t)((len + p.chunk - 1) / p.chunk);
+    return p;
+}
+
+template <int HD>
+void launch_stream_hd(dim3 grid, dim3 block, uint32_t gb, hipStream_t st, const uint16_t *q, const uint16_t *kc,
+                      const uint16_t *vc, uint32_t nh, uint32_t nkv, uint32_t len, uint32_t chunk, uint32_t hgw,
+                      float scale, float *part, uint16_t *out) {
+    const size_t lds = block.x / 64 * ATS_TILE * HD * 2;
+    if (gb == 4)
+        hipLaunchKernelGGL((attention_stream<HD, 4>), grid, block, lds, st, q, kc, vc, nh, nkv, len, chunk, hgw, scale,
+                           part, out);
+    else if (gb == 2)
+        hipLaunchKernelGGL((attention_stream<HD, 2>), grid, block, lds, st, q, kc, vc, nh, nkv, len, chunk, hgw, scale,
+                           part, out);
+    else
+        hipLaunchKernelGGL((attention_stream<HD, 1>), grid, block, lds, st, q, kc, vc, nh, nkv, len, chunk, hgw, scale,
+                           part, out);
+}
+
+int launch_stream(const uint16_t *q, const uint16_t *kc, const uint16_t *vc, size_t nh, size_t nkv, size_t hd,
+                  size_t len, AttnPlan p, float scale, float *part, uint16_t *out, hipStream_t st) {
+    // Four heads a wave once that still gives every CU a workgroup: fewer heads
+    // a wave read the rows again from L2, but short caches need the workgroups.
+    // The head groups of one key/value head share a workgroup where the splits
+    // alone fill the chip. Workgroups of four waves where two fit on every CU
+    // (their 64 KB of keys each), else of eight.
+    const size_t per_kv = nh / nkv, cus = (size_t)device_props().cus, tiles = (p.chunk + ATS_TILE - 1) / ATS_TILE;
+    uint32_t gb = 4;
+    while (gb > 1 && (gb / 2 >= per_kv || p.splits * nkv * ((per_kv + gb - 1) / gb) < cus)) gb /= 2;
+    const size_t hgroups = (per_kv + gb - 1) / gb;
+    size_t hgw = 1, waves = ATS_WAVES;
+    if (p.splits * nkv >= cus && hgroups > 1) hgw = hgroups > 2 ? 4 : 2;
+    else if (p.splits * nkv * hgroups >= 2 * cus) waves = ATS_WAVES / 2;
+    if (waves > tiles * hgw) waves = tiles * hgw;
+    const dim3 grid(p.splits, (unsigned)(nkv * ((hgroups + hgw - 1) / hgw))), block(64 * (unsigned)waves);
+    if (hd == 128)
+        launch_stream_hd<128>(grid, block, gb, st, q, kc, vc, (uint32_t)nh, (uint32_t)nkv, (uint32_t)len, p.chunk,
+                              (uint32_t)hgw, scale, part, out);
+    else
+        launch_stream_hd<64>(grid, block, gb, st, q, kc, vc, (uint32_t)nh, (uint32_t)nkv, (uint32_t)len, p.chunk,
+                             (uint32_t)hgw, scale, part, out);
+    return check_launch("attention_stream");
+}
+
 int launch_attention(const uint16_t *q, const uint16_t *kc, const uint16_t *vc, size_t nh, size_t nkv, size_t hd,
                      size_t len, float scale, float *part, uint16_t *out, hipStream_t st) {
-    const AttnPlan p = attn_plan(len, part != nullptr);
+    AttnPlan p = attn_plan(len, part != nullptr);
     const uint32_t gb = p.splits > 1 ? head_group(nh / nkv, p.splits, nh) : 1u;
     const size_t npairs = hd / 2, dpb = npairs < (size_t)ATT_THREADS ? npairs : (size_t)ATT_THREADS;
     const size_t lds = (ATT_THREADS / dpb) * gb * hd * sizeof(float);
@@ -679,7 +1009,11 @@ int launch_attention(const uint16_t *q, const uint16_t *kc, const uint16_t *vc, 
     const bool v16 = v8 && hd <= 128 && (reinterpret_cast<uintptr_t>(vc) & 15) == 0;
     float *wp = p.splits > 1 ? part : nullptr;
     const dim3 grid(p.splits, (unsigned)(nh / gb));
-    if (v16)
+    if (v16 && (hd == 64 || hd == 128) && nkv * hd <= ((size_t)1 << 24)) {
+        p = stream_plan(p, len);
+        wp = p.splits > 1 ? part : nullptr;
+        if (int rc = launch_stream(q, kc, vc, nh, nkv, hd, len, p, scale, wp, out, st)) return rc;
+    } else if (v16)
         hipLaunchKernelGGL(attention_split16, grid, dim3(ATT_THREADS), 0, st, q, kc, vc, (uint32_t)nh, (uint32_t)nkv,
                            (uint32_t)hd, (uint32_t)len, p.chunk, gb, scale, wp, out);
     else if (v8)

@@ -519,3 +519,36 @@ def test_attention_forms_against_numpy(nh, nkv, hd):
             kk[2:] = dk
             off = bf16_f32(bits(R.attention_decode_split(dq, kk[2:], dv, nh, nkv, hd, length, scale, workspace=ws)))
             assert O.rel_l2(off, want) < 4e-3, (length, "4-byte keys")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv,hd", [(5, 1, 128), (28, 4, 128), (7, 1, 64), (6, 2, 64), (12, 1, 128), (1, 1, 64)])
+def test_attention_stream_edges(nh, nkv, hd):
+    """The streaming kernel (head_dim 64, 128) at the edges of its 64-row tiles,
+    the one-pass limit and the splits, with head groups of every size (5 heads
+    are 4 + 1, 7 are 4 + 3, 12 three groups), cache rows past the length full
+    of NaN and keys whose scores are -infinity (weight 0; whole tiles of them).
+    The result is rounded to bf16 once: 2^-9 of a value at most, and the f32
+    sums stay below 1e-4."""
+    import torch
+
+    import reng_hip as R
+
+    rng = np.random.default_rng(nh * 1000 + hd)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    bits = lambda t: t.view(torch.int16).cpu().numpy().view(np.uint16)
+    scale = hd ** -0.5
+    for length, dead in ((1, 0), (63, 0), (64, 0), (65, 64), (511, 0), (512, 130), (513, 0), (1024, 1000), (1025, 0),
+                         (4161, 2500), (16500, 0)):
+        kb = bf16_bits(rng.standard_normal((length + 3, nkv * hd)).astype(np.float32) * 2)
+        vb = bf16_bits(rng.standard_normal((length + 3, nkv * hd)).astype(np.float32))
+        qb = bf16_bits(np.abs(rng.standard_normal(nh * hd)).astype(np.float32) + 2.0)
+        kb[:dead] = 0xff7f   # the most negative finite bf16
+        kb[length:] = vb[length:] = 0x7fc0
+        want = _attention_want(bf16_f32(qb), bf16_f32(kb[dead:length]), bf16_f32(vb[dead:length]), nh, nkv, hd, scale)
+        dq, dk, dv = dev(qb.view(np.int16)), dev(kb.view(np.int16).ravel()), dev(vb.view(np.int16).ravel())
+        ws = torch.full((R.attention_workspace_bytes(nh, hd, length) // 4 + 1,), float("nan"), device="cuda")
+        one = bf16_f32(bits(R.attention_decode(dq, dk, dv, nh, nkv, hd, length, scale)))
+        split = bf16_f32(bits(R.attention_decode_split(dq, dk, dv, nh, nkv, hd, length, scale, workspace=ws)))
+        assert O.rel_l2(one, want) < 2.0 ** -9 + 1e-4, (length, "one pass")
+        assert O.rel_l2(split, want) < 2.0 ** -9 + 1e-4, (length, "split")
