@@ -10,8 +10,8 @@
 // through global_load_lds_dwordx4 into an S-slot ring with the XOR-swizzled
 // 16-byte chunks of mfma_pipe.h. A wave reads its activation fragments as
 // bf16 (one ds_read_b128 per 32-row tile and 16-k step) and its code
-// fragments as 8 fp8 bytes (one ds_read_b64), decodes the codes to bf16 in
-// registers with v_cvt_scalef32_pk_bf16_fp8/bf8 (exact), and feeds both to the
+// fragments as fp8 bytes (one ds_read_b128 per two k-steps), decodes the codes
+// to bf16 in registers with v_cvt_scalef32_pk_bf16_fp8/bf8 (exact), and feeds both to the
 // MFMA with f32 accumulation; the per-channel scale is applied once per output
 // in the epilogue. The codes cross HBM once per tile row of the grid; tiles
 // run in XCD-major order with m fastest, so the blocks on one XCD that share
@@ -44,7 +44,7 @@ struct Tile {
     static constexpr int A_ROW = 2 * BK, B_ROW = BK;            // bytes of one activation / code row per stage
     static constexpr int CHA = A_ROW / 16, CHB = B_ROW / 16;    // 16-byte chunks of a row
     static constexpr int RA = 1024 / A_ROW, RB = 1024 / B_ROW;  // rows of a 1 KB copy
-    static constexpr int KSTEPS = BK / 16;                      // MFMA k-steps per stage
+    static constexpr int PAIRS = BK / 32;                       // pairs of 16-k MFMA k-steps per stage
     static constexpr int A_BYTES = BM * A_ROW, B_BYTES = BN * B_ROW, STAGE = A_BYTES + B_BYTES;
     static constexpr int LA = BM / RA / W, LB = BN / RB / W;    // copies per wave per stage
     static constexpr int LOADS = LA + LB;
@@ -94,8 +94,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void w8a16_tiles(const uint16_t *__
                                                               uint32_t vec_out, float *__restrict__ part,
                                                               uint32_t *__restrict__ cnt) {
     using T = Tile<WGM, WGN, WM, WN, BK>;
-    constexpr int BM = T::BM, BN = T::BN, NQ = WM * WN, HALF = NQ / 2;
-    constexpr int A_ROW = T::A_ROW, B_ROW = T::B_ROW, CHA = T::CHA, CHB = T::CHB, KSTEPS = T::KSTEPS;
+    constexpr int BM = T::BM, BN = T::BN, NQ = WM * WN;
+    constexpr int A_ROW = T::A_ROW, B_ROW = T::B_ROW, CHA = T::CHA, CHB = T::CHB, PAIRS = T::PAIRS;
     static_assert(S >= 2, "at least double-buffered");
     static_assert((S - 1) * T::LOADS < 64, "vmcnt range");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S * T::STAGE];
@@ -190,19 +190,33 @@ __global__ __launch_bounds__(64 * WGM * WGN) void w8a16_tiles(const uint16_t *__
         }
     };
 
-    // Fragments at k-step ks of a stage, lane l: row l % 32 of the 32-row tile
-    // and the 8 k of half h = l / 32: activation bytes 32 ks + 16 h (chunk
-    // 2 ks + h), codes bytes 16 ks + 8 h (chunk ks, second half for h = 1).
+    // Fragments come in pairs of k-steps (32 k). Lane l holds row l % 32 of a
+    // 32-row tile; half h = l / 32 has the 16 codes of chunk 2 p + h of pair p,
+    // the first 8 for its first k-step and the last 8 for its second, and the
+    // activations of the same k (chunks 4 p + 2 h and 4 p + 2 h + 1). Every read
+    // is a ds_read_b128 (8-byte code reads of one half of each chunk use half
+    // the banks), and a pair's reads have 2 WM WN MFMAs to land behind: with
+    // one k-step per fragment set the LDS latency (two waves per SIMD, one or
+    // two MFMAs each) showed in every k-step. One k-step -> pairs, same box:
+    // M = 256 [4096, 4096] 21.4 -> 18.2 us, [14336, 4096] 36.2 -> 33.8,
+    // [4096, 14336] 66.0 -> 60.1, M = 512 [5120, 5120] 40.0 -> 35.1, M = 1024
+    // [14336, 4096] 108 -> 105, [27648, 5120] 260 -> 249. (128 x 128 on four
+    // waves of 64 x 64, half the LDS reads: 39.0 against 37.6 us on M = 256
+    // [14336, 4096] past the Infinity Cache.)
     const uint32_t rl = lane & 31, h = lane >> 5, swa = swz_a(rl), swb = swz_b<CHB>(rl);
-    auto read_frags = [&](int slot, int ks, u32x4 (&fa)[WM], u32x2 (&fb)[WN]) __attribute__((always_inline)) {
+    auto read_pair = [&](int slot, int p, u32x4 (&fa)[2][WM], u32x4 (&fb)[WN]) __attribute__((always_inline)) {
         const uint8_t *base = lds + slot * T::STAGE;
-        const uint32_t oa = ((2 * ks + h) ^ swa) * 16, ob = ((uint32_t)ks ^ swb) * 16 + 8 * h;
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
-            fa[i] = *reinterpret_cast<const u32x4 *>(base + (wm * (32 * WM) + i * 32 + rl) * A_ROW + oa);
+        const uint32_t ob = ((2 * p + h) ^ swb) * 16;
 #pragma unroll
         for (int j = 0; j < WN; ++j)
-            fb[j] = *reinterpret_cast<const u32x2 *>(base + T::A_BYTES + (wn * (32 * WN) + j * 32 + rl) * B_ROW + ob);
+            fb[j] = *reinterpret_cast<const u32x4 *>(base + T::A_BYTES + (wn * (32 * WN) + j * 32 + rl) * B_ROW + ob);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const uint32_t oa = ((4 * p + 2 * h + ks) ^ swa) * 16;
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+                fa[ks][i] = *reinterpret_cast<const u32x4 *>(base + (wm * (32 * WM) + i * 32 + rl) * A_ROW + oa);
+        }
     };
 
     f32x16 acc[WM][WN];
@@ -216,22 +230,26 @@ __global__ __launch_bounds__(64 * WGM * WGN) void w8a16_tiles(const uint16_t *__
     };
     zero_acc();
 
-    // MFMAs q0 <= q < q1 of the wave's WM x WN tiles (q = i WN + j); the code
-    // fragments are decoded once per k-step. D = codes x^T: rows n, columns m.
-    auto mfma_part = [&](int q0, int q1, const u32x4 (&fa)[WM], const u32x4 (&wb)[WN]) __attribute__((always_inline)) {
+    // The MFMAs of a pair of k-steps; the code fragments are decoded as they
+    // are used. D = codes x^T: rows n, columns m.
+    auto mfma_pair = [&](const u32x4 (&fa)[2][WM], const u32x4 (&fb)[WN]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = q0; q < q1; ++q) {
-            const int i = q / WN, j = q % WN;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wb[j]),
-                                                                __builtin_bit_cast(bf16x8, fa[i]), acc[i][j], 0, 0,
-                                                                0);
+        for (int ks = 0; ks < 2; ++ks) {
+            u32x4 wb[WN];
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                const uint32_t lo = ks ? fb[j].z : fb[j].x, hi = ks ? fb[j].w : fb[j].y;
+                wb[j] = u32x4{dec_pair<F>(lo, false), dec_pair<F>(lo, true), dec_pair<F>(hi, false),
+                              dec_pair<F>(hi, true)};
+            }
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const int i = q / WN, j = q % WN;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wb[j]),
+                                                                    __builtin_bit_cast(bf16x8, fa[ks][i]), acc[i][j],
+                                                                    0, 0, 0);
+            }
         }
-    };
-    auto decode = [&](const u32x2 (&fb)[WN], u32x4 (&wb)[WN]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < WN; ++j)
-            wb[j] = u32x4{dec_pair<F>(fb[j].x, false), dec_pair<F>(fb[j].x, true), dec_pair<F>(fb[j].y, false),
-                          dec_pair<F>(fb[j].y, true)};
     };
 
     // Lane l holds output row m = ... + l % 32 and, per group g of four
@@ -398,36 +416,34 @@ __global__ __launch_bounds__(64 * WGM * WGN) void w8a16_tiles(const uint16_t *__
     for (int s = 0; s < S; ++s) issue(s);
     wait_vmcnt<(S - 1) * T::LOADS>();
     lds_barrier();
-    u32x4 fa[2][WM];
-    u32x2 fb[2][WN];
-    read_frags(0, 0, fa[0], fb[0]);
-    auto kstep = [&](auto cur_c, auto ks_c, uint32_t i) __attribute__((always_inline)) {
-        constexpr int CUR = decltype(cur_c)::value, NXT = CUR ^ 1, KSI = decltype(ks_c)::value;
-        u32x4 wb[WN];
-        decode(fb[CUR], wb);
-        if constexpr (KSI + 1 < KSTEPS) {
-            read_frags((int)(i % S), KSI + 1, fa[NXT], fb[NXT]);
-            mfma_part(0, NQ, fa[CUR], wb);
-            interleave<NQ, WM + WN, 0>();
+    u32x4 fa[2][2][WM], fb[2][WN];
+    read_pair(0, 0, fa[0], fb[0]);
+    // Pair PI of stage i on fragment set PI & 1, the next pair's fragments
+    // going into the other set. The stage's last pair starts with the barrier
+    // that publishes stage i + 1 and frees stage i's slot.
+    auto pair = [&](auto pi_c, uint32_t i) __attribute__((always_inline)) {
+        constexpr int PI = decltype(pi_c)::value, CUR = PI & 1, NXT = CUR ^ 1;
+        if constexpr (PI + 1 < PAIRS) {
+            read_pair((int)(i % S), PI + 1, fa[NXT], fb[NXT]);
+            mfma_pair(fa[CUR], fb[CUR]);
+            interleave<2 * NQ, 2 * WM + WN, 0>();
             __builtin_amdgcn_sched_barrier(0);
         } else {
-            mfma_part(0, HALF, fa[CUR], wb);
-            __builtin_amdgcn_sched_barrier(0);
+            wait_lgkm0();   // the stage's last fragments are in registers
             wait_vmcnt<(S - 2) * T::LOADS>();
             lds_barrier();
             issue((int)(i % S));
-            read_frags((int)((i + 1) % S), 0, fa[NXT], fb[NXT]);
-            mfma_part(HALF, NQ, fa[CUR], wb);
-            interleave<NQ - HALF, WM + WN, T::LOADS>();
+            read_pair((int)((i + 1) % S), 0, fa[NXT], fb[NXT]);
+            mfma_pair(fa[CUR], fb[CUR]);
+            interleave<2 * NQ, 2 * WM + WN, T::LOADS>();
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // k-step ks of every stage uses fragment set ks & 1 (KSTEPS is even).
-    static_assert(KSTEPS % 2 == 0, "the fragment sets alternate within a stage");
-    auto stage = [&](auto self, auto ks_c, uint32_t i) __attribute__((always_inline)) {
-        constexpr int KSI = decltype(ks_c)::value;
-        kstep(std::integral_constant<int, KSI & 1>{}, ks_c, i);
-        if constexpr (KSI + 1 < KSTEPS) self(self, std::integral_constant<int, KSI + 1>{}, i);
+    static_assert(PAIRS % 2 == 0, "the fragment sets alternate within a stage");
+    auto stage = [&](auto self, auto pi_c, uint32_t i) __attribute__((always_inline)) {
+        constexpr int PI = decltype(pi_c)::value;
+        pair(pi_c, i);
+        if constexpr (PI + 1 < PAIRS) self(self, std::integral_constant<int, PI + 1>{}, i);
     };
     // The block's units tile by tile: a run of stages, then the tile's end.
     uint32_t i = 0, f_t = t_first, f_ks = s_first;
