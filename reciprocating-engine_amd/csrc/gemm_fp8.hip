@@ -6,8 +6,9 @@
 // v_mfma_f32_32x32x64_f8f6f4 on the OCP fp8 formats, whose finite codes
 // 0x00-0x77 (e4m3) / 0x00-0x7b (e5m2) mean exactly what reng-fp8's codes mean.
 //
-// Two kernels: gemm_fp8_wide (further down) for shapes of whole 256 x 256 /
-// 256 x 128 tiles, and gemm_fp8_mfma for everything else. gemm_fp8_mfma:
+// Two kernels: gemm_fp8_wide (further down) for products of at least one tile
+// each way with N a multiple of 8, and gemm_fp8_mfma for everything else (fewer
+// than 64 rows or columns, N not a multiple of 8). gemm_fp8_mfma:
 // block = 2 x 2 waves; a wave owns WM x WN tiles of 32 x 32, so the block tile
 // is BM = 64 WM by BN = 64 WN. A pipeline stage covers BK = 64 KS codes of k.
 // Each stage's operand rows are copied global -> LDS by the waves'
@@ -286,8 +287,11 @@ int launch_fp8_cfg(const Fp8Args &g, hipStream_t st) {
 // buffer_load_dwordx4 ... lds through a buffer resource: the per-lane part of
 // the address (row within the copy, swizzled chunk) is one VGPR for every
 // copy of the wave, and the copy's row base and k offset ride in the scalar
-// soffset, so the copy addresses cost no registers. Only shapes that divide
-// into whole tiles take this form (every row read exists; no clamping).
+// soffset, so the copy addresses cost no registers. Every row read exists and
+// nothing is clamped: where M or N is not a whole number of tiles, the last
+// tile is moved back to end at the edge and computes some of its neighbour's
+// outputs again. An output's sum runs over the same stages and MFMA k-steps in
+// either tile, so both store the same bits.
 // Two waves per SIMD let one wave's MFMAs run while the other waits on its
 // fragment reads or the stage barrier; the 256 x 256 tile halves the operand
 // bytes each output needs against 128 x 128.
@@ -332,7 +336,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_fp8_wide(const uint8_t *_
     // operand rows per XCD.
     uint32_t mt, nt;
     wide_tile_of(blockIdx.x, tiles_m, tiles, mapm, mt, nt);
-    const uint32_t m0 = mt * BM, n0 = nt * BN;
+    // A tile past the edge moves back to end there (M >= BM, N >= BN: wide_fits).
+    const uint32_t m0 = mt * BM < M - BM ? mt * BM : M - BM, n0 = nt * BN < N - BN ? nt * BN : N - BN;
     const uint32_t n = K / BK;
 
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)a, 0, M * K, 0x00020000);
@@ -518,12 +523,13 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_fp8_wide(const uint8_t *_
     }
 }
 
-// Whether the wide (WM, WN) form takes this product: whole tiles, K in whole
-// stages, byte offsets in 31 bits, 16-byte aligned output rows.
+// Whether the wide (WM, WN) form takes this product: at least one tile each
+// way, K in whole stages, byte offsets in 31 bits, 16-byte aligned output rows
+// (of N, and of a wider output's ldo, both multiples of 8).
 template <int WM, int WN, int BK = 128, int WGM = 2, int WGN = 4>
 bool wide_fits(const Fp8Args &g) {
     using T = WideTile<WM, WN, BK, WGM, WGN>;
-    return g.M % T::BM == 0 && g.N % T::BN == 0 && g.K % T::BK == 0 && (uint64_t)g.M * g.K < (1ull << 31) &&
+    return g.M >= T::BM && g.N >= T::BN && g.N % 8 == 0 && g.K % T::BK == 0 && (uint64_t)g.M * g.K < (1ull << 31) &&
            (uint64_t)g.N * g.K < (1ull << 31) && reinterpret_cast<uintptr_t>(g.out) % 16 == 0;
 }
 
@@ -552,8 +558,9 @@ WideCand wide_cand(const Fp8Args &g, float c0, float c1) {
 template <int WM, int WN, int BK, int S, int WGM = 2, int WGN = 4>
 int launch_fp8_wide(const Fp8Args &g, hipStream_t st, uint32_t ldo = 0) {
     using T = WideTile<WM, WN, BK, WGM, WGN>;
-    const uint32_t tiles_m = g.M / T::BM, tiles = tiles_m * (g.N / T::BN);
-    const uint32_t mapm = wide_mapm(tiles_m, g.N / T::BN, T::BM, T::BN);
+    const uint32_t tiles_m = (g.M + T::BM - 1) / T::BM, tiles_n = (g.N + T::BN - 1) / T::BN;
+    const uint32_t tiles = tiles_m * tiles_n;
+    const uint32_t mapm = wide_mapm(tiles_m, tiles_n, T::BM, T::BN);
     const uint32_t ld = ldo ? ldo : g.N;
 #define RENG_FP8_WIDE(A, B)                                                                                      \
     hipLaunchKernelGGL((gemm_fp8_wide<A, B, WM, WN, BK, S, WGM, WGN>), dim3(tiles), dim3(64 * T::NW), 0, st, g.a, g.sa, \
@@ -602,15 +609,15 @@ inline MixedPlan mixed_plan(const Fp8Args &g, uint64_t cus, float c0a, float c1a
     using TA = WideTile<4, 2, 128, 2, 4>;
     using TB = WideTile<2, 3, 128, 4, 2>;
     MixedPlan best{0, 0.0f};
-    if (g.M % TA::BM != 0 || g.N % 64 != 0 || g.K % TA::BK != 0) return best;
-    const uint64_t tiles_m = g.M / TA::BM, stages = g.K / TA::BK;
+    if (g.M < TA::BM || g.N % 8 != 0 || g.K % TA::BK != 0) return best;
+    const uint64_t tiles_m = (g.M + TA::BM - 1) / TA::BM, stages = g.K / TA::BK;
     const uint64_t rounds_a = tiles_m * (g.N / TA::BN) / cus;   // whole rounds of the 256 x 256 tiles
     for (uint64_t r = 1; r <= rounds_a; ++r) {
         const uint64_t amax = r * cus / tiles_m;
         for (uint64_t a = amax; a + 3 > amax && a > 0; --a) {
             if (a * TA::BN >= g.N) continue;
             const uint64_t rest = g.N - a * TA::BN;
-            if (rest % TB::BN != 0 || tiles_m * (rest / TB::BN) > cus) continue;
+            if (rest < TB::BN || tiles_m * ((rest + TB::BN - 1) / TB::BN) > cus) continue;
             if (!wide_fits<4, 2, 128, 2, 4>(column_range(g, 0, (uint32_t)(a * TA::BN))) ||
                 !wide_fits<2, 3, 128, 4, 2>(column_range(g, (uint32_t)(a * TA::BN), (uint32_t)rest)))
                 continue;
@@ -630,7 +637,11 @@ int launch_fp8_gemm(const uint8_t *a, int fa, const float *sa, uint32_t nsa, con
     using namespace fp8gemm;
     const Fp8Args g{a, fa, sa, nsa, b, fb, sb, nsb, M, N, K, out};
     const uint64_t cus = (uint64_t)device_props().cus;
-    // Whole tiles: the wide forms. Each candidate's time is modelled as
+    // The wide forms, where at least a tile fits each way (ragged edges: the
+    // last tile moves back; same box against the clamped-row kernel [1000,
+    // 27648, 5120] 172 -> 134 us, [1000, 5120, 5120] 36.5 -> 29.5, [450, 20000,
+    // 1280] 28.2 -> 21.4, and against 64 x 64 tiles [1984, 4096, 4096] 71.5 ->
+    // 32.3). Each candidate's time is modelled as
     // rounds x (c0 + c1 x stages), rounds = ceil(tiles / CUs), stages = K / 128,
     // with (c0, c1) in microseconds fitted to timings of every form on eleven
     // products (M 256-2048, N 1024-27648, K 4096-27648; shorter K is an
@@ -648,7 +659,8 @@ int launch_fp8_gemm(const uint8_t *a, int fa, const float *sa, uint32_t nsa, con
     float best = 0.0f;
     for (int i = 0; i < (int)(sizeof(cands) / sizeof(cands[0])); ++i) {
         if (!cands[i].fits) continue;
-        const uint64_t tiles = (uint64_t)(M / cands[i].bm) * (N / cands[i].bn);
+        const uint64_t tiles =
+            (uint64_t)((M + cands[i].bm - 1) / cands[i].bm) * ((N + cands[i].bn - 1) / cands[i].bn);
         const float est = (float)((tiles + cus - 1) / cus) * (cands[i].c0 + cands[i].c1 * (float)(K / 128));
         if (pick < 0 || est < best) pick = i, best = est;
     }
@@ -658,6 +670,10 @@ int launch_fp8_gemm(const uint8_t *a, int fa, const float *sa, uint32_t nsa, con
         if (rc != RENG_HIP_OK) return rc;
         return launch_fp8_wide<2, 3, 128, 2, 4, 2>(column_range(g, mp.n1, N - mp.n1), st, N);
     }
+    // Where 64 x 64 tiles are the cheapest and do not divide the product, the
+    // clamped-row kernel below is faster ([100, 14336, 4096] 21.2 against
+    // 22.6 us, [130, 1000, 16384] 24.4 against 26.8).
+    if (pick == 4 && (M % 64 != 0 || N % 64 != 0)) pick = -1;
     switch (pick) {
     case 0: return launch_fp8_wide<4, 2, 128, 2>(g, st);
     case 1: return launch_fp8_wide<2, 2, 128, 3, 4, 2>(g, st);

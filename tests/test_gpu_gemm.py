@@ -555,6 +555,30 @@ def test_fp8_gemm_wide_tiles(R, M, N, K, fa, fb):
         check_fp8(R, rng, M, N, K, fa, fb, act, nsb, sample_cols=96)
 
 
+# M and N that no tile divides, down to one past a tile, over every wide form
+# (and the mixed grid, 1000 x 27640): tiles past the edge move back onto their
+# neighbour's outputs.
+@pytest.mark.parametrize("M,N,K", [(64, 72, 128), (65, 64, 256), (127, 1000, 384), (333, 4104, 640), (1000, 4104, 1024),
+                                   (1000, 5112, 1024), (520, 16392, 384), (1000, 16376, 256), (1000, 27640, 256)])
+def test_fp8_gemm_tiles_at_ragged_edges(R, M, N, K):
+    """Against the oracle, and bit for bit against the clamped-row kernel that
+    an output off 16-byte alignment takes: every sum runs over the same MFMA
+    k-steps in both."""
+    rng = np.random.default_rng(M + N + K)
+    check_fp8(R, rng, M, N, K, E4M3, E5M2, sample_cols=96)
+    a, b = (O.quantize(bf16_bits(rng.standard_normal((r, K)).astype(np.float32)).ravel(), r, K, E4M3, "pcs")
+            for r in (M, N))
+    both = []
+    for off in (0, 4):
+        y = torch.full((M * N + 8,), -1, dtype=torch.int16, device="cuda")
+        R.gemm_fp8_scaled(dev(a.codes), E4M3, dev(a.scales), dev(b.codes), E4M3, dev(b.scales), M, N, K,
+                          y[off:off + M * N].view(torch.bfloat16))
+        y = y.cpu().numpy()
+        assert (y[:off] == -1).all() and (y[off + M * N:] == -1).all()
+        both.append(y[off:off + M * N])
+    assert np.array_equal(*both)
+
+
 def test_fp8_gemm_every_output_of_a_qwen_32b_projection(R):
     """Every output of the M = 1024 prefill product on Qwen2.5-32B's q/o shape
     [5120, 5120], each element against float64 numpy."""
