@@ -43,7 +43,7 @@ int launch_skinny_mfma(const uint16_t *x, const uint8_t *codes, const float *sca
 // Up to 64 bf16 activation rows on skinny_wide (16 < M, or K % 128 != 0), K % 16 == 0 (csrc/skinny.hip).
 int launch_skinny_wide(const uint16_t *x, const uint8_t *codes, const float *scales, uint32_t M, uint32_t N,
                        uint32_t K, int format, uint16_t *y, hipStream_t st, const SplitScratch *fixed);
-// More than 64 activation rows, K % 64 == 0, on whole output tiles
+// More than 64 activation rows on output tiles
 // (csrc/gemm_tiles.hip). w8a16_tiles_take says whether the tiled kernel takes
 // the product (enough tiles for the chip; otherwise the 64-row kernels loop).
 bool w8a16_tiles_take(uint32_t M, uint32_t N, uint32_t K);

@@ -902,7 +902,7 @@ int launch_w8a16_t(const uint16_t *x, const uint8_t *codes, const float *scales,
     // More than 64 rows: output tiles on the bf16 MFMA, each code tile read
     // once per 64-256 activation rows (the 64-row loop below re-reads every
     // code once per 64 rows: M = 256 [14336, 4096] 86.8 -> 41.6 us).
-    if (M > 64 && K % 64 == 0 && w8a16_tiles_take(M, N, K))
+    if (M > 64 && w8a16_tiles_take(M, N, K))
         return launch_w8a16_tiles(x, codes, scales, M, N, K, F, y, st, fixed);
     if (M > 4 && K % 128 != 0) {
         // K not a multiple of the 128-code chunk: skinny_wide (its last chunk

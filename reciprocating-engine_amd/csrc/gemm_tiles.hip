@@ -33,7 +33,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int K_ALIGN = 64;   // K granularity the kernels take
+// What a copy past a row's end reads (TAIL).
+static __device__ const uint32_t zero_chunk[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
 
 // BK codes of k per pipeline stage (64, 128 or 256).
 template <int WGM, int WGN, int WM, int WN, int BK>
@@ -85,7 +86,12 @@ __device__ __forceinline__ uint32_t dec_pair<RENG_HIP_E5M2>(uint32_t w, bool hi)
 // order whichever block arrives last, so the sum is deterministic), writes the
 // tile and resets the counter to zero for the next launch. No block waits for
 // another.
-template <int F, int WGM, int WGN, int WM, int WN, int BK, int S, bool SK>
+//
+// With TAIL (no SK), K is any multiple of 16 and the last stage is short: a
+// lane whose 16-byte chunk lies past its row's end copies zeros instead, in
+// both operands, so the chunk adds exact zeros to the sums. The check costs a
+// compare and two selects per copy, so whole stages take the form without it.
+template <int F, int WGM, int WGN, int WM, int WN, int BK, int S, bool SK, bool TAIL>
 __global__ __launch_bounds__(64 * WGM * WGN) void w8a16_tiles(const uint16_t *__restrict__ x,
                                                               const uint8_t *__restrict__ codes,
                                                               const float *__restrict__ scales, uint32_t M,
@@ -98,12 +104,13 @@ __global__ __launch_bounds__(64 * WGM * WGN) void w8a16_tiles(const uint16_t *__
     constexpr int A_ROW = T::A_ROW, B_ROW = T::B_ROW, CHA = T::CHA, CHB = T::CHB, PAIRS = T::PAIRS;
     static_assert(S >= 2, "at least double-buffered");
     static_assert((S - 1) * T::LOADS < 64, "vmcnt range");
+    static_assert(!(SK && TAIL), "stream-K stages are whole");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S * T::STAGE];
     __shared__ uint32_t last_flag;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    const uint32_t n = K / BK;   // stages per tile
+    const uint32_t n = TAIL ? (K + BK - 1) / BK : K / BK;   // stages per tile
     const uint64_t U = (uint64_t)tiles * n, G = gridDim.x;
 
     uint64_t ub, ue;   // this block's units
@@ -160,11 +167,19 @@ __global__ __launch_bounds__(64 * WGM * WGN) void w8a16_tiles(const uint16_t *__
         if constexpr (!SK) {
             const uint32_t st = issued < L ? issued : L - 1;
             ++issued;
+            const uint8_t *zero = reinterpret_cast<const uint8_t *>(zero_chunk);
 #pragma unroll
-            for (int q = 0; q < T::LA; ++q) copy16_to_lds(ga[q] + (size_t)st * A_ROW, base + (wave * T::LA + q) * 1024);
+            for (int q = 0; q < T::LA; ++q) {
+                const uint8_t *src = ga[q] + (size_t)st * A_ROW;
+                if constexpr (TAIL) src = st * A_ROW + ofa[q] < 2 * K ? src : zero;
+                copy16_to_lds(src, base + (wave * T::LA + q) * 1024);
+            }
 #pragma unroll
-            for (int q = 0; q < T::LB; ++q)
-                copy16_to_lds(gb[q] + (size_t)st * B_ROW, base + T::A_BYTES + (wave * T::LB + q) * 1024);
+            for (int q = 0; q < T::LB; ++q) {
+                const uint8_t *src = gb[q] + (size_t)st * B_ROW;
+                if constexpr (TAIL) src = st * B_ROW + ofb[q] < K ? src : zero;
+                copy16_to_lds(src, base + T::A_BYTES + (wave * T::LB + q) * 1024);
+            }
             return;
         }
         const uint32_t m0 = c_tm * BM, n0 = c_tn * BN, st = c_ks;
@@ -460,7 +475,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void w8a16_tiles(const uint16_t *__
 // One launch; under SK, `part` holds (G + tiles - 1) BM BN floats and `cnt`
 // one zeroed counter per tile (left zeroed by the launch) for a grid of G
 // blocks.
-template <int F, int WGM, int WGN, int WM, int WN, int BK, int S, bool SK>
+template <int F, int WGM, int WGN, int WM, int WN, int BK, int S, bool SK, bool TAIL = false>
 int launch_tiles_cfg(const uint16_t *x, const uint8_t *codes, const float *scales, uint32_t M, uint32_t N,
                      uint32_t K, uint16_t *y, hipStream_t st, uint32_t grid, float *part, uint32_t *cnt) {
     using T = Tile<WGM, WGN, WM, WN, BK>;
@@ -470,7 +485,7 @@ int launch_tiles_cfg(const uint16_t *x, const uint8_t *codes, const float *scale
     // direct store of 8-byte groups, which this implies).
     const uint32_t vec_out = N % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
     if (!SK) grid = tiles;
-    hipLaunchKernelGGL((w8a16_tiles<F, WGM, WGN, WM, WN, BK, S, SK>), dim3(grid), dim3(64 * T::W), 0, st, x, codes,
+    hipLaunchKernelGGL((w8a16_tiles<F, WGM, WGN, WM, WN, BK, S, SK, TAIL>), dim3(grid), dim3(64 * T::W), 0, st, x, codes,
                        scales, M, N, K, tiles_m, tiles, y, vec_out, part, cnt);
     return check_launch("w8a16_tiles");
 }
@@ -497,6 +512,36 @@ inline bool streamk_suits(uint32_t M, uint32_t N, uint32_t K) {
 // M = 1024 [5120, 27648] 328 -> 308 us with 128 x 160). Stream-K takes
 // (G + tiles - 1) BM BN floats of partials (6.3 Mi floats at most on 256
 // CUs) and a counter per tile (fewer than 128).
+struct TilePick {
+    int form;
+    float est;   // modelled microseconds
+};
+
+inline TilePick tile_pick(uint32_t M, uint32_t N, uint32_t K) {
+    struct Cand {
+        uint32_t bm, bn;
+        float c0, c1;
+        bool fits;
+    };
+    const Cand cands[] = {
+        {256, 256, 28.6f, 1.130f, true},                            // 8 waves of 128 x 64, 64-code stages, 3 slots
+        {128, 256, 18.1f, 0.703f, true},                            // 8 waves of 64 x 64, 3 slots
+        {128, 160, 5.6f, 0.700f, K % 64 != 0 || K % 128 == 0},      // 4 waves of 32 x 160, 128-code stages, 2 slots
+        {128, 128, 10.2f, 0.465f, true},                            // 8 waves of 64 x 32, 6 slots
+        {64, 128, 5.0f, 0.348f, true},                              // 8 waves of 32 x 32, 6 slots
+        {64, 64, 0.0f, 0.251f, true},                               // 4 waves of 32 x 32, 6 slots
+    };
+    const uint64_t cus = (uint64_t)device_props().cus;
+    TilePick best{0, 0.0f};
+    for (int i = 0; i < 6; ++i) {
+        if (!cands[i].fits) continue;
+        const uint64_t rounds = (tile_count(M, N, cands[i].bm, cands[i].bn) + cus - 1) / cus;
+        const float est = (float)rounds * (cands[i].c0 + cands[i].c1 * (float)((K + 63) / 64));
+        if (i == 0 || est < best.est) best = TilePick{i, est};
+    }
+    return best;
+}
+
 template <int F>
 int launch_tiles_f(const uint16_t *x, const uint8_t *codes, const float *scales, uint32_t M, uint32_t N,
                    uint32_t K, uint16_t *y, hipStream_t st, const SplitScratch *fixed) {
@@ -514,45 +559,40 @@ int launch_tiles_f(const uint16_t *x, const uint8_t *codes, const float *scales,
         if (rc) return rc;
         return launch_tiles_cfg<F, 2, 4, 2, 1, 128, 3, true>(x, codes, scales, M, N, K, y, st, grid, part, cnt);
     }
-    struct Cand {
-        uint32_t bm, bn;
-        float c0, c1;
-        bool fits;
-    };
-    const Cand cands[] = {
-        {256, 256, 28.6f, 1.130f, true},            // 8 waves of 128 x 64, 64-code stages, 3 slots
-        {128, 256, 18.1f, 0.703f, true},            // 8 waves of 64 x 64, 3 slots
-        {128, 160, 5.6f, 0.700f, K % 128 == 0},     // 4 waves of 32 x 160, 128-code stages, 2 slots
-        {128, 128, 10.2f, 0.465f, true},            // 8 waves of 64 x 32, 6 slots
-        {64, 128, 5.0f, 0.348f, true},              // 8 waves of 32 x 32, 6 slots
-        {64, 64, 0.0f, 0.251f, true},               // 4 waves of 32 x 32, 6 slots
-    };
-    int pick = 0;
-    float best = 0.0f;
-    for (int i = 0; i < 6; ++i) {
-        if (!cands[i].fits) continue;
-        const uint64_t rounds = (tile_count(M, N, cands[i].bm, cands[i].bn) + cus - 1) / cus;
-        const float est = (float)rounds * (cands[i].c0 + cands[i].c1 * (float)(K / 64));
-        if (i == 0 || est < best) pick = i, best = est;
+    const bool tail = K % 64 != 0;   // a short last stage: every form takes it
+#define RENG_TILES(...)                                                                                          \
+    return tail ? launch_tiles_cfg<F, __VA_ARGS__, false, true>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr) \
+                : launch_tiles_cfg<F, __VA_ARGS__, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr)
+    switch (tile_pick(M, N, K).form) {
+    case 0: RENG_TILES(2, 4, 4, 2, 64, 3);
+    case 1: RENG_TILES(2, 4, 2, 2, 64, 3);
+    case 2: RENG_TILES(4, 1, 1, 5, 128, 2);
+    case 3: RENG_TILES(2, 4, 2, 1, 64, 6);
+    case 4: RENG_TILES(2, 4, 1, 1, 64, 6);
+    default: RENG_TILES(2, 2, 1, 1, 64, 6);
     }
-    switch (pick) {
-    case 0: return launch_tiles_cfg<F, 2, 4, 4, 2, 64, 3, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr);
-    case 1: return launch_tiles_cfg<F, 2, 4, 2, 2, 64, 3, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr);
-    case 2: return launch_tiles_cfg<F, 4, 1, 1, 5, 128, 2, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr);
-    case 3: return launch_tiles_cfg<F, 2, 4, 2, 1, 64, 6, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr);
-    case 4: return launch_tiles_cfg<F, 2, 4, 1, 1, 64, 6, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr);
-    default: return launch_tiles_cfg<F, 2, 2, 1, 1, 64, 6, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr);
-    }
+#undef RENG_TILES
 }
 
 }  // namespace tiles
 
-// Below half the CUs in 64 x 128 tiles the 64-row kernels, which split K,
-// are faster (M = 100 [3000, 4096]: 22.2 against 28.1 us) - unless the
-// product suits stream-K.
+// K % 64 == 0: below half the CUs in 64 x 128 tiles the 64-row kernels, which
+// split K, are faster (M = 100 [3000, 4096]: 22.2 against 28.1 us) - unless
+// the product suits stream-K. K no multiple of 128: the 64-row launches, each
+// about 6 us + N K / 2.9 TB/s there (M = 128 [14336, 4112] 25 us a launch,
+// M = 300 [3000, 3600] 10, M = 700 [1500, 1296] 7.4), against the tiles' own
+// model, a quarter added for the short stage's checks and few tiles (M = 70
+// [4000, 6160]: tiles 30.8 us, two launches 27.7). M = 256 [4096, 4112] 54.1 ->
+// 22.7 us, M = 300 [3000, 3600] 50.2 -> 20.7, M = 1000 [10000, 1552] 174 -> 51,
+// M = 1024 [2048, 16400] 340 -> 105.
 bool w8a16_tiles_take(uint32_t M, uint32_t N, uint32_t K) {
-    return M > 64 && K % tiles::K_ALIGN == 0 &&
-           (tiles::streamk_suits(M, N, K) || 2 * tiles::tile_count(M, N, 64, 128) >= (uint64_t)device_props().cus);
+    if (M <= 64) return false;
+    if (K % 64 == 0 &&
+        (tiles::streamk_suits(M, N, K) || 2 * tiles::tile_count(M, N, 64, 128) >= (uint64_t)device_props().cus))
+        return true;
+    if (K % 128 == 0) return false;
+    const float loop = (float)((M + 63) / 64) * (6.0f + (float)N * (float)K / 2.9e6f);
+    return 1.25f * tiles::tile_pick(M, N, K).est < loop;
 }
 
 int launch_w8a16_tiles(const uint16_t *x, const uint8_t *codes, const float *scales, uint32_t M, uint32_t N,

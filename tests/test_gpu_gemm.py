@@ -441,6 +441,30 @@ def test_w8a16_tiles_every_output(R, M, N, K, fmt):
 
 
 @pytest.mark.parametrize("M, N, K, fmt", [
+    (1024, 16390, 80, E4M3),    # 256 x 256 tiles; a short second stage
+    (520, 16300, 144, E5M2),    # 128 x 256 tiles; one chunk in the last stage
+    (1000, 5100, 176, E4M3),    # 128 x 160 tiles; 48 codes past a whole stage
+    (768, 4097, 1552, E5M2),    # 128 x 128 tiles; ragged N
+    (200, 4097, 3120, E4M3),    # 64 x 128 tiles
+    (96, 8192, 16, E5M2),       # 64 x 64 tiles; one chunk in all
+])
+def test_w8a16_tiles_short_last_stage(R, M, N, K, fmt):
+    """More than 64 activation rows and K a multiple of 16 but not of 64: the
+    tiled kernel's last stage is padded with zeros. x and the codes are views
+    that end in NaNs, so a chunk read past a row's end would show."""
+    rng = np.random.default_rng(M * 5 + N + K)
+    check_w8a16(R, rng, M, N, K, fmt)
+    q = quantized_weight(rng, N, K, fmt)
+    x = bf16_bits(rng.standard_normal((M, K)).astype(np.float32)).ravel()
+    outs = []
+    for pad in (0, 256):
+        xp = np.concatenate([x, np.full(pad, 0x7fc0, np.uint16)])
+        cp = np.concatenate([q.codes, np.full(pad, 0x7f, np.uint8)])
+        outs.append(R.gemm_w8a16(dev(xp)[:M * K], dev(cp)[:N * K], dev(q.scales), M, N, K, fmt).view(torch.int16))
+    assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("M, N, K, fmt", [
     (256, 2048, 8192, E4M3),    # 32 tiles of 128 x 128 over 64 stages each: stream-K
     (200, 1000, 8320, E5M2),    # ragged M and N under stream-K
 ])
