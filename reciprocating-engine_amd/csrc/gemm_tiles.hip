@@ -5,8 +5,8 @@
 // rows crates/reng-model/src/bin/fp8_probe.rs:359-431 times).
 //
 // Output tiles of BM x BN on v_mfma_f32_32x32x16_bf16: a block of WGM x WGN
-// waves, each owning WM x WN tiles of 32 x 32. Per 64-k stage the activation
-// rows (128 bytes each) and the code rows (64 bytes each) go global -> LDS
+// waves, each owning WM x WN tiles of 32 x 32. Per stage of BK k (64 or 128)
+// the activation rows (2 BK bytes each) and the code rows (BK bytes each) go global -> LDS
 // through global_load_lds_dwordx4 into an S-slot ring with the XOR-swizzled
 // 16-byte chunks of mfma_pipe.h. A wave reads its activation fragments as
 // bf16 (one ds_read_b128 per 32-row tile and 16-k step) and its code
@@ -506,10 +506,11 @@ inline bool streamk_suits(uint32_t M, uint32_t N, uint32_t K) {
 // rounds x (c0 + c1 x K / 64), rounds = ceil(tiles / CUs), with (c0, c1) in
 // microseconds fitted to graph-replayed timings of every form on eleven
 // products (M 128-1024 over the Llama-3.1-8B and Qwen2.5-32B shapes; most
-// within 16% of the fit), and the cheapest form runs; on those products that
-// is the fastest one measured (M = 256 [4096, 4096] 26.6 -> 21.8 us with
-// 64 x 64 tiles, M = 512 [5120, 5120] 64.4 -> 43.2 us with 128 x 128,
-// M = 1024 [5120, 27648] 328 -> 308 us with 128 x 160). Stream-K takes
+// within 16% of the fit), scaled per form to this pipeline's times (0.91-0.93;
+// 256 x 256 and 64 x 64 1.06-1.08), and the cheapest form runs. On 22 products
+// (M 80-1024, N 1200-28672, K 1024-10240) the picks were all faster than
+// those of the earlier fit and pipeline, by 4-33% (M = 700 [3000, 2048] 25.5
+// -> 17.3 us, M = 150 [25000, 1536] 31.0 -> 23.4). Stream-K takes
 // (G + tiles - 1) BM BN floats of partials (6.3 Mi floats at most on 256
 // CUs) and a counter per tile (fewer than 128).
 struct TilePick {
@@ -524,12 +525,12 @@ inline TilePick tile_pick(uint32_t M, uint32_t N, uint32_t K) {
         bool fits;
     };
     const Cand cands[] = {
-        {256, 256, 28.6f, 1.130f, true},                            // 8 waves of 128 x 64, 64-code stages, 3 slots
-        {128, 256, 18.1f, 0.703f, true},                            // 8 waves of 64 x 64, 3 slots
-        {128, 160, 5.6f, 0.700f, K % 64 != 0 || K % 128 == 0},      // 4 waves of 32 x 160, 128-code stages, 2 slots
-        {128, 128, 10.2f, 0.465f, true},                            // 8 waves of 64 x 32, 6 slots
-        {64, 128, 5.0f, 0.348f, true},                              // 8 waves of 32 x 32, 6 slots
-        {64, 64, 0.0f, 0.251f, true},                               // 4 waves of 32 x 32, 6 slots
+        {256, 256, 28.6f, 1.200f, true},                            // 8 waves of 128 x 64, 64-code stages, 3 slots
+        {128, 256, 16.6f, 0.650f, true},                            // 8 waves of 64 x 64
+        {128, 160, 5.2f, 0.650f, K % 64 != 0 || K % 128 == 0},      // 4 waves of 32 x 160, 128-code stages, 2 slots
+        {128, 128, 9.3f, 0.425f, true},                             // 8 waves of 64 x 32, 64-code stages, 6 slots
+        {64, 128, 4.6f, 0.318f, true},                              // 8 waves of 32 x 32
+        {64, 64, 0.0f, 0.270f, true},                               // 4 waves of 32 x 32
     };
     const uint64_t cus = (uint64_t)device_props().cus;
     TilePick best{0, 0.0f};
@@ -563,14 +564,25 @@ int launch_tiles_f(const uint16_t *x, const uint8_t *codes, const float *scales,
 #define RENG_TILES(...)                                                                                          \
     return tail ? launch_tiles_cfg<F, __VA_ARGS__, false, true>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr) \
                 : launch_tiles_cfg<F, __VA_ARGS__, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr)
+    // Whole 128-code stages copy the codes in 128-byte pieces rather than 64
+    // (of L2-resident rows a CU takes in 125 GB/s of the former, 69-93 of the
+    // latter). Same box, 64- against 128-code stages: 128 x 256 M = 512 [14336,
+    // 4096] 60.8 -> 58.0 us, 64 x 128 M = 128 [14336, 4096] 27.2 -> 24.9, 64 x 64
+    // M = 256 [4096, 4096] 18.2 -> 17.3 (three slots: two blocks fit a CU; six:
+    // 18.0). The 128 x 128 form needs the six slots (M = 512 [5120, 5120] 34.6
+    // against 37.8 us), and 256 x 256 of 128-code stages does not fit.
+    const bool wide = K % 128 == 0;
+#define RENG_TILES_128(...)                                                                                      \
+    return launch_tiles_cfg<F, __VA_ARGS__, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr)
     switch (tile_pick(M, N, K).form) {
     case 0: RENG_TILES(2, 4, 4, 2, 64, 3);
-    case 1: RENG_TILES(2, 4, 2, 2, 64, 3);
+    case 1: if (wide) RENG_TILES_128(2, 4, 2, 2, 128, 2); RENG_TILES(2, 4, 2, 2, 64, 3);
     case 2: RENG_TILES(4, 1, 1, 5, 128, 2);
     case 3: RENG_TILES(2, 4, 2, 1, 64, 6);
-    case 4: RENG_TILES(2, 4, 1, 1, 64, 6);
-    default: RENG_TILES(2, 2, 1, 1, 64, 6);
+    case 4: if (wide) RENG_TILES_128(2, 4, 1, 1, 128, 4); RENG_TILES(2, 4, 1, 1, 64, 6);
+    default: if (wide) RENG_TILES_128(2, 2, 1, 1, 128, 3); RENG_TILES(2, 2, 1, 1, 64, 6);
     }
+#undef RENG_TILES_128
 #undef RENG_TILES
 }
 

@@ -441,6 +441,17 @@ def test_w8a16_tiles_every_output(R, M, N, K, fmt):
 
 
 @pytest.mark.parametrize("M, N, K, fmt", [
+    (520, 16300, 256, E4M3),    # 128 x 256 tiles over two stages, ragged M and N
+    (200, 4097, 1152, E5M2),    # 64 x 128 tiles, more stages than slots
+    (130, 8190, 128, E4M3),     # one stage
+    (96, 8200, 384, E5M2),      # 64 x 64 tiles, as many stages as slots
+])
+def test_w8a16_tiles_of_128_code_stages(R, M, N, K, fmt):
+    """K a multiple of 128: the narrower tile forms stage 128 codes at a time."""
+    check_w8a16(R, np.random.default_rng(M * 3 + N + K), M, N, K, fmt)
+
+
+@pytest.mark.parametrize("M, N, K, fmt", [
     (1024, 16390, 80, E4M3),    # 256 x 256 tiles; a short second stage
     (520, 16300, 144, E5M2),    # 128 x 256 tiles; one chunk in the last stage
     (1000, 5100, 176, E4M3),    # 128 x 160 tiles; 48 codes past a whole stage
