@@ -273,9 +273,9 @@ RENG_HIP_API int reng_hip_rope_append(uint16_t *q, const uint16_t *k, const uint
 /* One query per head over cache rows 0 .. len - 1 (layer_cpu's causal attention,
  * model.rs:3010-3050): out[h] = softmax(scale * q[h] . K[:, g]) V[:, g] with
  * g = h / (n_heads / n_kv_heads), bf16 in and out, f32 inside (online softmax
- * over tiles of 256 rows); 1 <= len <= RENG_HIP_ATTENTION_MAX_LEN; q, k_cache
+ * over tiles of rows); 1 <= len <= RENG_HIP_ATTENTION_MAX_LEN; q, k_cache
  * and v_cache 4-byte aligned. One workgroup per query head reads the whole
- * cache: for caches past 512 rows use reng_hip_attention_decode_split. */
+ * cache: for longer caches use reng_hip_attention_decode_split. */
 RENG_HIP_API int reng_hip_attention_decode(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v_cache,
                                            size_t n_heads, size_t n_kv_heads, size_t head_dim, size_t len,
                                            float scale, uint16_t *out, void *stream);
