@@ -563,8 +563,9 @@ __device__ __forceinline__ float row16_sum_all(float v) {
     return v;
 }
 
-// exp(v - m), and 0 where m is -infinity: nothing but -infinity scores so far.
-__device__ __forceinline__ float exp_from(float v, float m) { return m == -INFINITY ? 0.0f : expf(v - m); }
+// exp(v - m), and 0 where v is -infinity, whatever m is. It is v that is tested: m leaves NaN out
+// (fmaxf), so a NaN score may meet an m of -infinity and has to come out as NaN.
+__device__ __forceinline__ float exp_from(float v, float m) { return v == -INFINITY ? 0.0f : expf(v - m); }
 
 // 16 bytes per lane from r at off into LDS at l + 16 * lane (l wave-uniform).
 __device__ __forceinline__ void buf_copy16_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t off, uint8_t *l) {

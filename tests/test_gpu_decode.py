@@ -552,3 +552,49 @@ def test_attention_stream_edges(nh, nkv, hd):
         split = bf16_f32(bits(R.attention_decode_split(dq, dk, dv, nh, nkv, hd, length, scale, workspace=ws)))
         assert O.rel_l2(one, want) < 2.0 ** -9 + 1e-4, (length, "one pass")
         assert O.rel_l2(split, want) < 2.0 ** -9 + 1e-4, (length, "split")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 128), (32, 8, 128), (28, 4, 64), (8, 2, 96)])
+def test_attention_keeps_nan(nh, nkv, hd):
+    """A NaN key makes its score NaN, and a NaN score makes the whole softmax
+    NaN: every output of the query heads that read the key, wherever it lies
+    among the 16 rows, 64-row tiles and splits that meet before any other score
+    is known (the newest key alone past a multiple of 16, blocks of 16 and of 64
+    from a multiple). A NaN value makes its own dimension NaN. The heads of the
+    other key/value heads keep their bits. (8, 2, 96) is the general kernel."""
+    import torch
+
+    import reng_hip as R
+
+    rng = np.random.default_rng(nh * 1000 + hd)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    bits = lambda t: t.view(torch.int16).cpu().numpy().view(np.uint16).reshape(nh, hd)
+    g0, per = nkv - 1, nh // nkv
+    mine = slice(g0 * per, (g0 + 1) * per)
+    for length in (1, 17, 33, 65, 513, 1025, 4161):
+        q = dev(bf16_bits(rng.standard_normal(nh * hd).astype(np.float32)).view(np.int16))
+        k = dev(bf16_bits(rng.standard_normal((length, nkv * hd)).astype(np.float32)).view(np.int16))
+        v = dev(bf16_bits(rng.standard_normal((length, nkv * hd)).astype(np.float32)).view(np.int16))
+        ws = torch.empty(R.attention_workspace_bytes(nh, hd, length) // 4 + 1, device="cuda")
+        forms = (lambda kk, vv: bits(R.attention_decode(q, kk, vv, nh, nkv, hd, length, hd ** -0.5)),
+                 lambda kk, vv: bits(R.attention_decode_split(q, kk, vv, nh, nkv, hd, length, hd ** -0.5,
+                                                              workspace=ws)))
+        clean = [f(k, v) for f in forms]
+        mid = length // 2 // 64 * 64
+        for rows in {(length - 1, length), (0, 1), (length // 2, length // 2 + 1), (0, 16), (mid, mid + 16),
+                     (mid, mid + 64), (0, length)}:
+            bad = k.clone()
+            bad[rows[0]:rows[1], g0 * hd + 5] = 0x7fc0
+            for f, want in zip(forms, clean):
+                got = f(bad, v)
+                assert np.isnan(bf16_f32(got[mine])).all(), (length, rows)
+                got[mine] = want[mine]
+                assert np.array_equal(got, want), (length, rows)
+        bad = v.clone()
+        bad[length - 1, g0 * hd + 7] = 0x7fc0
+        for f, want in zip(forms, clean):
+            got = f(k, bad)
+            assert np.isnan(bf16_f32(got[mine, 7])).all(), length
+            got[mine, 7] = want[mine, 7]
+            assert np.array_equal(got, want), length
