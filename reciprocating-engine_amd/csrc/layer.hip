@@ -17,6 +17,7 @@
 // residual stream is f32; what feeds a GEMV is bf16 (the w8a16 contract).
 // These are latency-bound per token (a few KB each); only the GEMVs stream
 // HBM.
+#include "attention_plan.h"
 #include "common.h"
 #include "mfma_pipe.h"
 
@@ -134,7 +135,6 @@ __global__ __launch_bounds__(64) void rope_append(uint16_t *__restrict__ q, cons
 // writes bf16(o / l); otherwise the unnormalised o and (m, l) of its split go
 // to the workspace and attention_combine merges the splits.
 constexpr int ATT_NW = 16, ATT_THREADS = 64 * ATT_NW, ATT_TILE = 16 * ATT_NW, ATT_GMAX = 4;
-constexpr int ATT_SPLIT_MAX = 64, ATT_SPLIT_ROWS = 256, ATT_ONE_PASS_MAX = 512;
 constexpr int ATT_VPF = 16;   // value rows per thread requested with the tile's keys
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -142,21 +142,6 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float acc) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), acc,
                                            false);
-}
-
-struct AttnPlan {
-    uint32_t splits, chunk;
-};
-
-// One pass (S = 1) for caches of up to 512 rows or without a workspace; else
-// S = min(64, ceil(len / 256)) splits of equal length (the last one shorter),
-// none empty.
-inline AttnPlan attn_plan(size_t len, bool split) {
-    if (!split || len <= (size_t)ATT_ONE_PASS_MAX) return {1u, (uint32_t)len};
-    size_t s = (len + ATT_SPLIT_ROWS - 1) / ATT_SPLIT_ROWS;
-    if (s > (size_t)ATT_SPLIT_MAX) s = ATT_SPLIT_MAX;
-    const size_t chunk = (len + s - 1) / s;
-    return {(uint32_t)((len + chunk - 1) / chunk), (uint32_t)chunk};
 }
 
 __device__ __forceinline__ float wave_max_f32(float v) {
@@ -545,8 +530,6 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_split16(
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-constexpr int ATS_TILE = 64, ATS_WAVES = 8, ATS_ONE_PASS_MAX = 1024;
-
 template <int CTRL>
 __device__ __forceinline__ float row16_max_step(float v) {
     return fmaxf(v, dpp_mov<CTRL, 0xf>(v));
@@ -613,7 +596,7 @@ __device__ __forceinline__ void accumulate_rows(const float (&p)[4], const Value
 template <int HD, int GB>
 __global__ __launch_bounds__(64 * ATS_WAVES) void attention_stream(
     const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc, uint32_t nh,
-    uint32_t nkv, uint32_t len, uint32_t chunk, uint32_t hgw, float scale, float *__restrict__ part,
+    uint32_t nkv, uint32_t len, StreamSplit sp, uint32_t hgw, float scale, float *__restrict__ part,
     uint16_t *__restrict__ out) {
     constexpr int STEPS = HD / 32, DPL = HD / 16, N = GB * DPL;
     constexpr int CH = HD / 8, STAGE = ATS_TILE * HD * 2;   // 16-byte chunks of a row; bytes of a tile's keys
@@ -624,13 +607,16 @@ __global__ __launch_bounds__(64 * ATS_WAVES) void attention_stream(
     const uint32_t slots = (blockDim.x >> 6) / hgw;   // tiles side by side
     const uint32_t s = blockIdx.x, per_kv = nh / nkv;
     // y walks the key/value heads fastest: the groups of one sit gridDim.x *
-    // nkv workgroups apart, on one XCD when that is a multiple of 8, and share
-    // its rows in L2.
+    // nkv workgroups apart, on one XCD when that is a multiple of 8, and share its
+    // rows in L2. stream_launch passes the splits for it: a workgroup past them has
+    // no rows and stores nothing (a return here would put three rounds of argument
+    // loads in a row: 0.2 us).
     const uint32_t g = blockIdx.y % nkv, hb = blockIdx.y / nkv * hgw * GB;   // the workgroup's first head of g
     const uint32_t hg = hb + wave % hgw * GB;                                // the wave's
     const uint32_t hn = hg < per_kv ? min((uint32_t)GB, per_kv - hg) : 0;
     const uint32_t pitch = nkv * HD * 2;   // bytes
-    const uint32_t j0 = s * chunk, j1 = min(len, j0 + chunk);
+    const uint32_t j0 = (s * sp.tiles + min(s, sp.more)) * ATS_TILE;
+    const uint32_t j1 = min(len, j0 + (sp.tiles + (s < sp.more)) * ATS_TILE);
 
     bf16x8_t qv[STEPS];
     const uint16_t *qh = q + (size_t)(g * per_kv + (hn ? hg + min(l16 & 3, hn - 1) : 0)) * HD + 8 * lg;
@@ -761,7 +747,7 @@ __global__ __launch_bounds__(64 * ATS_WAVES) void attention_stream(
     }
     __syncthreads();
     // The waves.
-    const uint32_t heads = min(hgw * GB, per_kv - hb), h0 = g * per_kv + hb;
+    const uint32_t heads = s < sp.splits ? min(hgw * GB, per_kv - hb) : 0, h0 = g * per_kv + hb;
     for (uint32_t i = tid; i < heads * HD; i += blockDim.x) {
         const uint32_t h = i / HD % GB, w0 = i / HD / GB;
         float M = mw[w0][h];
@@ -778,7 +764,7 @@ __global__ __launch_bounds__(64 * ATS_WAVES) void attention_stream(
         } else {
             part[((size_t)s * nh + h0) * HD + i] = v;
             if (i % HD == 0) {
-                float *ml = part + (size_t)gridDim.x * nh * HD;
+                float *ml = part + (size_t)sp.splits * nh * HD;
                 ml[((size_t)s * nh + h0 + i / HD) * 2] = M;
                 ml[((size_t)s * nh + h0 + i / HD) * 2 + 1] = ls;
             }
@@ -947,56 +933,32 @@ int attention_args(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v
     return RENG_HIP_OK;
 }
 
-// Whole tiles per split, so that no wave runs a part-filled one but the last:
-// never more splits than attn_plan's, whose workspace they use. One pass up to
-// 1024 rows, where the merge's launch costs more than the split saves (one
-// pass / split, 32 heads on 8 of 128 dimensions: 7.1 / 9.1 us at 768 rows, 9.0
-// / 9.7 at 1024, 25 / 12 at 4096; 8 heads on 2 of 64: 6.5 / 8.2 at 1024).
-AttnPlan stream_plan(AttnPlan p, size_t len) {
-    if (p.splits < 2 || len <= (size_t)ATS_ONE_PASS_MAX) return {1u, (uint32_t)len};
-    p.chunk = (p.chunk + ATS_TILE - 1) / ATS_TILE * ATS_TILE;
-    p.splits = (uint32_t)((len + p.chunk - 1) / p.chunk);
-    return p;
-}
-
 template <int HD>
 void launch_stream_hd(dim3 grid, dim3 block, uint32_t gb, hipStream_t st, const uint16_t *q, const uint16_t *kc,
-                      const uint16_t *vc, uint32_t nh, uint32_t nkv, uint32_t len, uint32_t chunk, uint32_t hgw,
+                      const uint16_t *vc, uint32_t nh, uint32_t nkv, uint32_t len, StreamSplit sp, uint32_t hgw,
                       float scale, float *part, uint16_t *out) {
     const size_t lds = block.x / 64 * ATS_TILE * HD * 2;
     if (gb == 4)
-        hipLaunchKernelGGL((attention_stream<HD, 4>), grid, block, lds, st, q, kc, vc, nh, nkv, len, chunk, hgw, scale,
+        hipLaunchKernelGGL((attention_stream<HD, 4>), grid, block, lds, st, q, kc, vc, nh, nkv, len, sp, hgw, scale,
                            part, out);
     else if (gb == 2)
-        hipLaunchKernelGGL((attention_stream<HD, 2>), grid, block, lds, st, q, kc, vc, nh, nkv, len, chunk, hgw, scale,
+        hipLaunchKernelGGL((attention_stream<HD, 2>), grid, block, lds, st, q, kc, vc, nh, nkv, len, sp, hgw, scale,
                            part, out);
     else
-        hipLaunchKernelGGL((attention_stream<HD, 1>), grid, block, lds, st, q, kc, vc, nh, nkv, len, chunk, hgw, scale,
+        hipLaunchKernelGGL((attention_stream<HD, 1>), grid, block, lds, st, q, kc, vc, nh, nkv, len, sp, hgw, scale,
                            part, out);
 }
 
 int launch_stream(const uint16_t *q, const uint16_t *kc, const uint16_t *vc, size_t nh, size_t nkv, size_t hd,
-                  size_t len, AttnPlan p, float scale, float *part, uint16_t *out, hipStream_t st) {
-    // Four heads a wave once that still gives every CU a workgroup: fewer heads
-    // a wave read the rows again from L2, but short caches need the workgroups.
-    // The head groups of one key/value head share a workgroup where the splits
-    // alone fill the chip. Workgroups of four waves where two fit on every CU
-    // (their 64 KB of keys each), else of eight.
-    const size_t per_kv = nh / nkv, cus = (size_t)device_props().cus, tiles = (p.chunk + ATS_TILE - 1) / ATS_TILE;
-    uint32_t gb = 4;
-    while (gb > 1 && (gb / 2 >= per_kv || p.splits * nkv * ((per_kv + gb - 1) / gb) < cus)) gb /= 2;
-    const size_t hgroups = (per_kv + gb - 1) / gb;
-    size_t hgw = 1, waves = ATS_WAVES;
-    if (p.splits * nkv >= cus && hgroups > 1) hgw = hgroups > 2 ? 4 : 2;
-    else if (p.splits * nkv * hgroups >= 2 * cus) waves = ATS_WAVES / 2;
-    if (waves > tiles * hgw) waves = tiles * hgw;
-    const dim3 grid(p.splits, (unsigned)(nkv * ((hgroups + hgw - 1) / hgw))), block(64 * (unsigned)waves);
+                  size_t len, StreamSplit sp, float scale, float *part, uint16_t *out, hipStream_t st) {
+    const StreamLaunch l = stream_launch(sp, nh, nkv, (size_t)device_props().cus);
+    const dim3 grid(l.gx, l.gy), block(64 * l.waves);
     if (hd == 128)
-        launch_stream_hd<128>(grid, block, gb, st, q, kc, vc, (uint32_t)nh, (uint32_t)nkv, (uint32_t)len, p.chunk,
-                              (uint32_t)hgw, scale, part, out);
+        launch_stream_hd<128>(grid, block, l.gb, st, q, kc, vc, (uint32_t)nh, (uint32_t)nkv, (uint32_t)len, sp,
+                              l.hgw, scale, part, out);
     else
-        launch_stream_hd<64>(grid, block, gb, st, q, kc, vc, (uint32_t)nh, (uint32_t)nkv, (uint32_t)len, p.chunk,
-                             (uint32_t)hgw, scale, part, out);
+        launch_stream_hd<64>(grid, block, l.gb, st, q, kc, vc, (uint32_t)nh, (uint32_t)nkv, (uint32_t)len, sp,
+                             l.hgw, scale, part, out);
     return check_launch("attention_stream");
 }
 
@@ -1011,9 +973,10 @@ int launch_attention(const uint16_t *q, const uint16_t *kc, const uint16_t *vc, 
     float *wp = p.splits > 1 ? part : nullptr;
     const dim3 grid(p.splits, (unsigned)(nh / gb));
     if (v16 && (hd == 64 || hd == 128) && nkv * hd <= ((size_t)1 << 24)) {
-        p = stream_plan(p, len);
+        const StreamSplit sp = stream_split(p.splits, len);
+        p.splits = sp.splits;
         wp = p.splits > 1 ? part : nullptr;
-        if (int rc = launch_stream(q, kc, vc, nh, nkv, hd, len, p, scale, wp, out, st)) return rc;
+        if (int rc = launch_stream(q, kc, vc, nh, nkv, hd, len, sp, scale, wp, out, st)) return rc;
     } else if (v16)
         hipLaunchKernelGGL(attention_split16, grid, dim3(ATT_THREADS), 0, st, q, kc, vc, (uint32_t)nh, (uint32_t)nkv,
                            (uint32_t)hd, (uint32_t)len, p.chunk, gb, scale, wp, out);

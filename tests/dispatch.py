@@ -1,0 +1,25 @@
+"""The launchers' choices, from the headers that the launchers themselves use
+(tests/cpp/dispatch.cpp)."""
+import ctypes
+import os
+import subprocess
+
+CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
+CUS = 256   # an MI355X
+_lib = None
+
+
+def lib():
+    global _lib
+    if _lib is None:
+        subprocess.run(["make", "-C", CPP, "build/libdispatch.so"], check=True, capture_output=True)
+        _lib = ctypes.CDLL(os.path.join(CPP, "build", "libdispatch.so"))
+        _lib.attention_stream_plan.argtypes = [ctypes.c_size_t] * 3 + [ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p]
+        _lib.attention_splits.argtypes = [ctypes.c_size_t]
+    return _lib
+
+
+def attention_stream_plan(nh, nkv, length, split=True, cus=CUS):
+    out = (ctypes.c_uint32 * 8)()
+    lib().attention_stream_plan(nh, nkv, length, int(split), cus, out)
+    return dict(zip(("splits", "tiles", "more", "gb", "hgw", "waves", "gx", "gy"), out))

@@ -1,0 +1,37 @@
+"""The launchers' choices on an MI355X's 256 CUs, on the host."""
+import pytest
+
+import dispatch as D
+
+LENGTHS = [1, 63, 64, 65, 512, 513, 1024, 1025, 1500, 3000, 6000, 12000, 16000, 16384, 16385, 20000, 32768, 70000,
+           131071, 131072]
+
+
+@pytest.mark.parametrize("nh,nkv", [(1, 1), (8, 1), (16, 1), (8, 2), (14, 2), (28, 4), (32, 8), (40, 8), (128, 8),
+                                    (32, 32), (20, 1)])
+def test_attention_stream_plan(nh, nkv):
+    """Every tile in one split and the splits even, as many as the workspace is
+    sized for past 1024 rows; every query head in one wave's group; whole groups
+    of waves; and, over several splits, the head groups of a key/value head on one XCD
+    (workgroup number mod 8)."""
+    per = nh // nkv
+    for split in (False, True):
+        for length in LENGTHS:
+            p = D.attention_stream_plan(nh, nkv, length, split)
+            tiles = -(-length // 64)
+            assert p["splits"] * p["tiles"] + p["more"] == tiles and p["more"] < p["splits"] and p["tiles"] >= 1
+            want = D.lib().attention_splits(length) if split and length > 1024 else 1
+            assert p["splits"] == want, (length, p)
+            if split and length > 63 * 256:
+                assert p["splits"] == 64, (length, p)
+            assert p["splits"] <= p["gx"] < p["splits"] + 8
+            assert p["waves"] % p["hgw"] == 0 and 0 < p["waves"] <= 8
+            groups = -(-per // p["gb"])
+            assert p["gy"] == nkv * -(-groups // p["hgw"]), (length, p)
+            heads = [y // nkv * p["hgw"] * p["gb"] + w * p["gb"] for y in range(0, p["gy"], nkv)
+                     for w in range(p["hgw"])]
+            assert sorted(h for h in heads if h < per) == list(range(0, per, p["gb"])), (length, p)
+            if p["splits"] > 1:
+                for s in range(p["splits"]):
+                    for g in range(nkv):
+                        assert len({(s + p["gx"] * y) % 8 for y in range(g, p["gy"], nkv)}) == 1, (length, p)
