@@ -7,8 +7,10 @@
 // 0x00-0x77 (e4m3) / 0x00-0x7b (e5m2) mean exactly what reng-fp8's codes mean.
 //
 // Two kernels: gemm_fp8_wide (further down) for products of at least one tile
-// each way with N a multiple of 8, and gemm_fp8_mfma for everything else (fewer
-// than 64 rows or columns, N not a multiple of 8). gemm_fp8_mfma:
+// each way with N a multiple of 8 and 16-byte aligned output, and gemm_fp8_mfma
+// for everything else (fewer than 64 rows or columns, N not a multiple of 8, a
+// misaligned output) and for products that the cheapest wide tile does not divide
+// where one of its forms is cheaper (fp8_pick, fp8_forms.h). gemm_fp8_mfma:
 // block = 2 x 2 waves; a wave owns WM x WN tiles of 32 x 32, so the block tile
 // is BM = 64 WM by BN = 64 WN. A pipeline stage covers BK = 64 KS codes of k.
 // Each stage's operand rows are copied global -> LDS by the waves'
@@ -29,6 +31,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "fp8_forms.h"
 #include "gemm.h"
 #include "mfma_pipe.h"
 #include "tile_order.h"
@@ -336,7 +339,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_fp8_wide(const uint8_t *_
     // operand rows per XCD.
     uint32_t mt, nt;
     wide_tile_of(blockIdx.x, tiles_m, tiles, mapm, mt, nt);
-    // A tile past the edge moves back to end there (M >= BM, N >= BN: wide_fits).
+    // A tile past the edge moves back to end there (M >= BM, N >= BN: fp8_wide_fits).
     const uint32_t m0 = mt * BM < M - BM ? mt * BM : M - BM, n0 = nt * BN < N - BN ? nt * BN : N - BN;
     const uint32_t n = K / BK;
 
@@ -523,30 +526,6 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_fp8_wide(const uint8_t *_
     }
 }
 
-// Whether the wide (WM, WN) form takes this product: at least one tile each
-// way, K in whole stages, byte offsets in 31 bits, 16-byte aligned output rows
-// (of N, and of a wider output's ldo, both multiples of 8).
-template <int WM, int WN, int BK = 128, int WGM = 2, int WGN = 4>
-bool wide_fits(const Fp8Args &g) {
-    using T = WideTile<WM, WN, BK, WGM, WGN>;
-    return g.M >= T::BM && g.N >= T::BN && g.N % 8 == 0 && g.K % T::BK == 0 && (uint64_t)g.M * g.K < (1ull << 31) &&
-           (uint64_t)g.N * g.K < (1ull << 31) && reinterpret_cast<uintptr_t>(g.out) % 16 == 0;
-}
-
-// A wide form as a dispatch candidate: whether it takes the product, its
-// tile, and its fitted time model (c0, c1).
-struct WideCand {
-    bool fits;
-    uint32_t bm, bn;
-    float c0, c1;
-};
-
-template <int WM, int WN, int WGM, int WGN>
-WideCand wide_cand(const Fp8Args &g, float c0, float c1) {
-    using T = WideTile<WM, WN, 128, WGM, WGN>;
-    return WideCand{wide_fits<WM, WN, 128, WGM, WGN>(g), (uint32_t)T::BM, (uint32_t)T::BN, c0, c1};
-}
-
 // 2-D XCD blocks of tiles (wide_mapm, tile_order.h): on the kv projection
 // [1024, 1024, 5120] (64 x 64 tiles: 16 m-tiles of which an XCD's run of 32
 // covers all, plus 2 n-tiles) blocks of 4 x 8 read 768 operand rows per XCD
@@ -573,6 +552,14 @@ int launch_fp8_wide(const Fp8Args &g, hipStream_t st, uint32_t ldo = 0) {
     return check_launch("gemm_fp8_wide");
 }
 
+// The tiles fp8_pick prices, in the launches' template arguments.
+static_assert(WideTile<4, 2, 128, 2, 4>::BM == 256 && WideTile<4, 2, 128, 2, 4>::BN == 256, "FP8_WIDE_256x256");
+static_assert(WideTile<2, 2, 128, 4, 2>::BM == 256 && WideTile<2, 2, 128, 4, 2>::BN == 128, "FP8_WIDE_256x128");
+static_assert(WideTile<1, 5, 128, 4, 1>::BM == 128 && WideTile<1, 5, 128, 4, 1>::BN == 160, "FP8_WIDE_128x160");
+static_assert(WideTile<2, 2, 128, 2, 2>::BM == 128 && WideTile<2, 2, 128, 2, 2>::BN == 128, "FP8_WIDE_128x128");
+static_assert(WideTile<1, 1, 128, 2, 2>::BM == 64 && WideTile<1, 1, 128, 2, 2>::BN == 64, "FP8_WIDE_64x64");
+static_assert(WideTile<2, 3, 128, 4, 2>::BM == 256 && WideTile<2, 3, 128, 4, 2>::BN == 192, "FP8_WIDE_MIXED's second");
+
 // The columns [n0, n0 + n) of a product as a product of its own: the codes and
 // per-channel scales of those weight rows, the output's columns from n0 (the
 // launch writes them with the whole output's row stride).
@@ -588,47 +575,6 @@ inline Fp8Args column_range(const Fp8Args &g, uint32_t n0, uint32_t n) {
     return r;
 }
 
-// A grid of 256 x 256 tiles that is not a whole number of rounds pays for its
-// last, partial round in full. The mixed plan runs whole rounds of 256 x 256
-// tiles over the leading n1 columns, then one round of 256 x 192 tiles over
-// the rest (a second launch): on [1024, 27648, 5120] 252 + 240 tiles instead of
-// 432 in two rounds. The narrower tile reads 0.875x the operand rows per output
-// and its round measured 0.82-0.85x as long, so the plan gains 2-3% there
-// (141-146 -> 138-141 us; K = 10240: 260-263 -> 253-254 us), not the 16% of a
-// tile-count model: these tiles' rounds take time in proportion to the operand
-// bytes they copy. (One launch holding both forms, the second's workgroups
-// dispatched as the first's finish, measured the same as two launches.)
-// n1 = 0: no plan. est uses the 256 x 192 form's (c0, c1) fitted to its
-// timings at K = 2560, 5120 and 10240.
-struct MixedPlan {
-    uint32_t n1;
-    float est;
-};
-
-inline MixedPlan mixed_plan(const Fp8Args &g, uint64_t cus, float c0a, float c1a, float c0b, float c1b) {
-    using TA = WideTile<4, 2, 128, 2, 4>;
-    using TB = WideTile<2, 3, 128, 4, 2>;
-    MixedPlan best{0, 0.0f};
-    if (g.M < TA::BM || g.N % 8 != 0 || g.K % TA::BK != 0) return best;
-    const uint64_t tiles_m = (g.M + TA::BM - 1) / TA::BM, stages = g.K / TA::BK;
-    const uint64_t rounds_a = tiles_m * (g.N / TA::BN) / cus;   // whole rounds of the 256 x 256 tiles
-    for (uint64_t r = 1; r <= rounds_a; ++r) {
-        const uint64_t amax = r * cus / tiles_m;
-        for (uint64_t a = amax; a + 3 > amax && a > 0; --a) {
-            if (a * TA::BN >= g.N) continue;
-            const uint64_t rest = g.N - a * TA::BN;
-            if (rest < TB::BN || tiles_m * ((rest + TB::BN - 1) / TB::BN) > cus) continue;
-            if (!wide_fits<4, 2, 128, 2, 4>(column_range(g, 0, (uint32_t)(a * TA::BN))) ||
-                !wide_fits<2, 3, 128, 4, 2>(column_range(g, (uint32_t)(a * TA::BN), (uint32_t)rest)))
-                continue;
-            const float est = (float)((tiles_m * a + cus - 1) / cus) * (c0a + c1a * (float)stages) +
-                              (c0b + c1b * (float)stages);
-            if (best.n1 == 0 || est < best.est) best = MixedPlan{(uint32_t)(a * TA::BN), est};
-        }
-    }
-    return best;
-}
-
 }  // namespace fp8gemm
 
 int launch_fp8_gemm(const uint8_t *a, int fa, const float *sa, uint32_t nsa, const uint8_t *b, int fb,
@@ -636,60 +582,22 @@ int launch_fp8_gemm(const uint8_t *a, int fa, const float *sa, uint32_t nsa, con
                     hipStream_t st) {
     using namespace fp8gemm;
     const Fp8Args g{a, fa, sa, nsa, b, fb, sb, nsb, M, N, K, out};
-    const uint64_t cus = (uint64_t)device_props().cus;
-    // The wide forms, where at least a tile fits each way (ragged edges: the
-    // last tile moves back; same box against the clamped-row kernel [1000,
-    // 27648, 5120] 172 -> 134 us, [1000, 5120, 5120] 36.5 -> 29.5, [450, 20000,
-    // 1280] 28.2 -> 21.4, and against 64 x 64 tiles [1984, 4096, 4096] 71.5 ->
-    // 32.3). Each candidate's time is modelled as
-    // rounds x (c0 + c1 x stages), rounds = ceil(tiles / CUs), stages = K / 128,
-    // with (c0, c1) in microseconds fitted to timings of every form on eleven
-    // products (M 256-2048, N 1024-27648, K 4096-27648; shorter K is an
-    // extrapolation). Most timings lie within 10% of the fit, 64 x 64 and
-    // 256 x 128 up to 26% above it when their tiles take a single round. The
-    // cheapest form runs; on those products that is the fastest one measured.
-    const WideCand cands[] = {
-        wide_cand<4, 2, 2, 4>(g, 16.2f, 1.318f),   // 256 x 256, 8 waves, 2 slots
-        wide_cand<2, 2, 4, 2>(g, 12.2f, 0.739f),   // 256 x 128, 8 waves, 3 slots
-        wide_cand<1, 5, 4, 1>(g, 8.6f, 0.658f),    // 128 x 160, 4 waves, 3 slots
-        wide_cand<2, 2, 2, 2>(g, 6.5f, 0.550f),    // 128 x 128, 4 waves, 3 slots
-        wide_cand<1, 1, 2, 2>(g, 1.1f, 0.246f),    // 64 x 64, 4 waves, 4 slots
-    };
-    int pick = -1;
-    float best = 0.0f;
-    for (int i = 0; i < (int)(sizeof(cands) / sizeof(cands[0])); ++i) {
-        if (!cands[i].fits) continue;
-        const uint64_t tiles =
-            (uint64_t)((M + cands[i].bm - 1) / cands[i].bm) * ((N + cands[i].bn - 1) / cands[i].bn);
-        const float est = (float)((tiles + cus - 1) / cus) * (cands[i].c0 + cands[i].c1 * (float)(K / 128));
-        if (pick < 0 || est < best) pick = i, best = est;
+    const Fp8Pick p = fp8_pick(M, N, K, reinterpret_cast<uintptr_t>(out) % 16 == 0, (uint64_t)device_props().cus);
+    switch (p.form) {
+    case FP8_WIDE_256x256: return launch_fp8_wide<4, 2, 128, 2>(g, st);
+    case FP8_WIDE_256x128: return launch_fp8_wide<2, 2, 128, 3, 4, 2>(g, st);
+    case FP8_WIDE_128x160: return launch_fp8_wide<1, 5, 128, 3, 4, 1>(g, st);
+    case FP8_WIDE_128x128: return launch_fp8_wide<2, 2, 128, 3, 2, 2>(g, st);
+    case FP8_WIDE_64x64: return launch_fp8_wide<1, 1, 128, 4, 2, 2>(g, st);
+    case FP8_WIDE_MIXED: {
+        const int rc = launch_fp8_wide<4, 2, 128, 2>(column_range(g, 0, p.n1), st, N);
+        return rc != RENG_HIP_OK ? rc : launch_fp8_wide<2, 3, 128, 2, 4, 2>(column_range(g, p.n1, N - p.n1), st, N);
     }
-    const MixedPlan mp = mixed_plan(g, cus, cands[0].c0, cands[0].c1, 8.2f, 1.353f);
-    if (mp.n1 != 0 && (pick < 0 || mp.est < best)) {
-        const int rc = launch_fp8_wide<4, 2, 128, 2>(column_range(g, 0, mp.n1), st, N);
-        if (rc != RENG_HIP_OK) return rc;
-        return launch_fp8_wide<2, 3, 128, 2, 4, 2>(column_range(g, mp.n1, N - mp.n1), st, N);
+    case FP8_ROWS_256x256: return launch_fp8_cfg<4, 4, 2, 2>(g, st);
+    case FP8_ROWS_256x128: return launch_fp8_cfg<4, 2, 2, 3>(g, st);
+    case FP8_ROWS_128x128: return launch_fp8_cfg<2, 2, 2, 2>(g, st);
+    case FP8_ROWS_64x64: break;
     }
-    // Where 64 x 64 tiles are the cheapest and do not divide the product, the
-    // clamped-row kernel below is faster ([100, 14336, 4096] 21.2 against
-    // 22.6 us, [130, 1000, 16384] 24.4 against 26.8).
-    if (pick == 4 && (M % 64 != 0 || N % 64 != 0)) pick = -1;
-    switch (pick) {
-    case 0: return launch_fp8_wide<4, 2, 128, 2>(g, st);
-    case 1: return launch_fp8_wide<2, 2, 128, 3, 4, 2>(g, st);
-    case 2: return launch_fp8_wide<1, 5, 128, 3, 4, 1>(g, st);
-    case 3: return launch_fp8_wide<2, 2, 128, 3, 2, 2>(g, st);
-    case 4: return launch_fp8_wide<1, 1, 128, 4, 2, 2>(g, st);
-    default: break;
-    }
-    // Ragged shapes: by how many tiles each size gives for the chip (measured
-    // on the M = 1024 prefill shapes): the largest tile that still fills every
-    // CU; 256 x 128 for long K; 64 x 64 for small outputs.
-    const uint64_t t256 = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
-    const uint64_t t128 = (uint64_t)((M + 127) / 128) * ((N + 127) / 128);
-    if (t256 >= cus) return launch_fp8_cfg<4, 4, 2, 2>(g, st);
-    if (t128 >= cus) return K > 8192 ? launch_fp8_cfg<4, 2, 2, 3>(g, st) : launch_fp8_cfg<2, 2, 2, 2>(g, st);
-    if (K > 8192 && 2 * t128 >= cus) return launch_fp8_cfg<4, 2, 2, 3>(g, st);
     return launch_fp8_cfg<1, 1, 2, 4>(g, st);
 }
 

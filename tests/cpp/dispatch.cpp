@@ -1,6 +1,7 @@
 // The launchers' choices (plain C++ headers of reciprocating-engine_amd/csrc)
 // for tests/test_dispatch.py and for the GPU tests that name a kernel form.
 #include "../../reciprocating-engine_amd/csrc/attention_plan.h"
+#include "../../reciprocating-engine_amd/csrc/fp8_forms.h"
 
 using namespace reng;
 
@@ -13,3 +14,7 @@ extern "C" void attention_stream_plan(size_t nh, size_t nkv, size_t len, int spl
 }
 
 extern "C" uint32_t attention_splits(size_t len) { return attn_plan(len, true).splits; }
+
+extern "C" int fp8_form(uint32_t M, uint32_t N, uint32_t K, int aligned, uint64_t cus) {
+    return fp8_pick(M, N, K, aligned != 0, cus).form;
+}

@@ -6,6 +6,8 @@ import subprocess
 
 CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
 CUS = 256   # an MI355X
+FP8_FORMS = ("wide 256x256", "wide 256x128", "wide 128x160", "wide 128x128", "wide 64x64", "wide mixed", "rows 256x256",
+             "rows 256x128", "rows 128x128", "rows 64x64")
 _lib = None
 
 
@@ -15,6 +17,7 @@ def lib():
         subprocess.run(["make", "-C", CPP, "build/libdispatch.so"], check=True, capture_output=True)
         _lib = ctypes.CDLL(os.path.join(CPP, "build", "libdispatch.so"))
         _lib.attention_stream_plan.argtypes = [ctypes.c_size_t] * 3 + [ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p]
+        _lib.fp8_form.argtypes = [ctypes.c_uint32] * 3 + [ctypes.c_int, ctypes.c_uint64]
         _lib.attention_splits.argtypes = [ctypes.c_size_t]
     return _lib
 
@@ -23,3 +26,8 @@ def attention_stream_plan(nh, nkv, length, split=True, cus=CUS):
     out = (ctypes.c_uint32 * 8)()
     lib().attention_stream_plan(nh, nkv, length, int(split), cus, out)
     return dict(zip(("splits", "tiles", "more", "gb", "hgw", "waves", "gx", "gy"), out))
+
+
+def fp8_form(M, N, K, aligned=True, cus=CUS):
+    """The form of an fp8 x fp8 product; aligned: its output starts on 16 bytes."""
+    return FP8_FORMS[lib().fp8_form(M, N, K, int(aligned), cus)]

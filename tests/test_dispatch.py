@@ -35,3 +35,18 @@ def test_attention_stream_plan(nh, nkv):
                 for s in range(p["splits"]):
                     for g in range(nkv):
                         assert len({(s + p["gx"] * y) % 8 for y in range(g, p["gy"], nkv)}) == 1, (length, p)
+
+
+@pytest.mark.parametrize("M,N,K,form", [
+    # The clamped-row kernel where no wide tile divides the product and it is ahead: two 128 x 128
+    # workgroups on a CU, and 256 x 128 for short M over long K.
+    (271, 19624, 3328, "rows 128x128"), (560, 11144, 4864, "rows 128x128"), (324, 20696, 3968, "rows 128x128"),
+    (136, 25912, 10752, "rows 256x128"),
+    # Beside them, and on whole tiles, the wide forms.
+    (1000, 5120, 5120, "wide 128x160"), (1000, 27648, 5120, "wide mixed"), (322, 16384, 1536, "wide 256x128"),
+    (1024, 1024, 5120, "wide 64x64"), (1024, 5120, 5120, "wide 128x160"), (1024, 27648, 5120, "wide mixed"),
+    (256, 19456, 3328, "wide 128x160"), (1773, 3784, 640, "wide 256x128"), (512, 11264, 4864, "wide 256x128"),
+])
+def test_fp8_forms(M, N, K, form):
+    assert D.fp8_form(M, N, K) == form
+    assert D.fp8_form(M, N, K, aligned=False).startswith("rows")
