@@ -2,6 +2,7 @@
 import pytest
 
 import dispatch as D
+import test_gpu_gemm as G
 
 LENGTHS = [1, 63, 64, 65, 512, 513, 1024, 1025, 1500, 3000, 6000, 12000, 16000, 16384, 16385, 20000, 32768, 70000,
            131071, 131072]
@@ -50,3 +51,15 @@ def test_attention_stream_plan(nh, nkv):
 def test_fp8_forms(M, N, K, form):
     assert D.fp8_form(M, N, K) == form
     assert D.fp8_form(M, N, K, aligned=False).startswith("rows")
+
+
+@pytest.mark.parametrize("M,N,K,form", G.FP8_WIDE + G.FP8_RAGGED)
+def test_fp8_test_shapes_run_the_forms_they_name(M, N, K, form):
+    assert D.fp8_form(M, N, K) == form
+    assert M % 64 == 0 and N % 64 == 0 if (M, N, K, form) in G.FP8_WIDE else M % 64 != 0 or N % 64 != 0
+
+
+def test_fp8_test_shapes_run_every_wide_form():
+    wide = {f for f in D.FP8_FORMS if f.startswith("wide")}
+    assert {c[3] for c in G.FP8_WIDE} == wide
+    assert {c[3] for c in G.FP8_RAGGED} & wide == wide - {"wide 64x64"}

@@ -576,13 +576,14 @@ def test_fp8_gemm_ragged_tiles(R, M, N, K):
 
 
 # Whole-tile shapes take the wide forms, one shape per tile the launcher's
-# cost model picks on a 256-CU MI355X: 256 x 256 (1024 x 16384), 256 x 128
-# (512 x 16384), 128 x 160 (1024 x 5120), 128 x 128 (1024 x 4096), 64 x 64
-# (256 x 32768), and the mixed grid (1024 x 27648: 252 tiles of 256 x 256 over
+# cost model picks on a 256-CU MI355X (the mixed grid: 252 tiles of 256 x 256 over
 # the first 16128 columns, 240 of 256 x 192 over the rest); K of one to eight
 # 128-code stages, every format pair and scale form.
-@pytest.mark.parametrize("M,N,K", [(1024, 16384, 256), (512, 16384, 384), (1024, 5120, 1024), (1024, 4096, 1024),
-                                   (256, 32768, 128), (1024, 27648, 256)])
+FP8_WIDE = [(1024, 16384, 256, "wide 256x256"), (512, 16384, 384, "wide 256x128"), (1024, 5120, 1024, "wide 128x160"),
+            (1024, 4096, 1024, "wide 128x128"), (256, 32768, 128, "wide 64x64"), (1024, 27648, 256, "wide mixed")]
+
+
+@pytest.mark.parametrize("M,N,K", [c[:3] for c in FP8_WIDE])
 @pytest.mark.parametrize("fa,fb", [(E4M3, E4M3), (E5M2, E5M2), (E4M3, E5M2), (E5M2, E4M3)])
 def test_fp8_gemm_wide_tiles(R, M, N, K, fa, fb):
     rng = np.random.default_rng(M + N + K + 4 * fa + fb)
@@ -590,15 +591,21 @@ def test_fp8_gemm_wide_tiles(R, M, N, K, fa, fb):
         check_fp8(R, rng, M, N, K, fa, fb, act, nsb, sample_cols=96)
 
 
-# M and N that no tile divides, down to one past a tile, over every wide form
-# (and the mixed grid, 1000 x 27640): tiles past the edge move back onto their
-# neighbour's outputs.
-@pytest.mark.parametrize("M,N,K", [(64, 72, 128), (65, 64, 256), (127, 1000, 384), (333, 4104, 640), (1000, 4104, 1024),
-                                   (1000, 5112, 1024), (520, 16392, 384), (1000, 16376, 256), (1000, 27640, 256)])
+# M and N that no tile divides, over every wide form but 64 x 64: tiles past the
+# edge move back onto their neighbour's outputs. Where 64 x 64 tiles or a form of
+# the clamped-row kernel are the cheapest, that kernel runs ("rows"), down to one
+# row or column past a tile.
+FP8_RAGGED = [(1000, 16376, 256, "wide 256x256"), (330, 13800, 1152, "wide 256x128"), (1000, 4104, 1024, "wide 128x160"),
+              (1000, 5112, 1024, "wide 128x160"), (203, 13008, 1024, "wide 128x128"), (1000, 27640, 256, "wide mixed"),
+              (64, 72, 128, "rows 64x64"), (65, 64, 256, "rows 64x64"), (127, 1000, 384, "rows 64x64"),
+              (333, 4104, 640, "rows 64x64"), (520, 16392, 384, "rows 128x128"), (262, 11288, 1024, "rows 128x128")]
+
+
+@pytest.mark.parametrize("M,N,K", [c[:3] for c in FP8_RAGGED])
 def test_fp8_gemm_tiles_at_ragged_edges(R, M, N, K):
     """Against the oracle, and bit for bit against the clamped-row kernel that
     an output off 16-byte alignment takes: every sum runs over the same MFMA
-    k-steps in both."""
+    k-steps in both (the rows forms differ from it in the tile at most)."""
     rng = np.random.default_rng(M + N + K)
     check_fp8(R, rng, M, N, K, E4M3, E5M2, sample_cols=96)
     a, b = (O.quantize(bf16_bits(rng.standard_normal((r, K)).astype(np.float32)).ravel(), r, K, E4M3, "pcs")
