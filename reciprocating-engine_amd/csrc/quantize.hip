@@ -153,8 +153,15 @@ __device__ __forceinline__ void store_scale(const QMat &M, uint64_t row, float s
 
 // How a row's vectors lie: every lane full (no tail predication), any count, or
 // any count, width and alignment (elements past the last whole vector one per
-// thread; 16-byte loads and code stores at whatever address).
-enum { ROWS_TAIL = 0, ROWS_FULL = 1, ROWS_ANY = 2 };
+// thread; 16-byte loads and code stores at whatever address). ROWS_SHARED is
+// ROWS_ANY for rows of up to 64 vectors that end inside a line: most of a row's
+// code lines are shared with the rows beside it, in other workgroups, and a
+// non-temporal store sends each part of a line out by itself; plain stores meet
+// in L2 (bf16 [605, 10] 4.5 -> 3.4 us, where quantize_rows_generic takes 3.5;
+// [4096, 33] 5.1 -> 4.5, [65536, 9] 26.1 -> 24.1). Whole lines and wider rows
+// keep the non-temporal ones ([16000, 512] off its input's alignment 9.1 us
+// against 9.5, [4096, 4001] 12.4 against 13.1).
+enum { ROWS_TAIL = 0, ROWS_FULL = 1, ROWS_ANY = 2, ROWS_SHARED = 3 };
 
 // One row per workgroup (WAVES waves) at a time, VPT 16-byte vectors per thread
 // held in registers between the absmax and the encode. Below ROWS_ANY it requires
@@ -165,7 +172,7 @@ enum { ROWS_TAIL = 0, ROWS_FULL = 1, ROWS_ANY = 2 };
 // narrower width 36, 41 and 46: a wave's 16-byte loads then cover no extra line).
 template <typename InT, int F, int VPT, int WAVES, bool CLAMP, int MODE>
 __global__ __launch_bounds__(64 * WAVES) void quantize_rows_fast(QBatch B, int scheme, float full) {
-    constexpr bool FULL = MODE == ROWS_FULL, ANY = MODE == ROWS_ANY;
+    constexpr bool FULL = MODE == ROWS_FULL, ANY = MODE >= ROWS_ANY;
     using IT = InTraits<InT>;
     constexpr int EPV = IT::EPV;
     constexpr int CPV = EPV / 4;                 // code dwords per vector: 2 (bf16), 1 (f32)
@@ -288,10 +295,11 @@ __global__ __launch_bounds__(64 * WAVES) void quantize_rows_fast(QBatch B, int s
             const int i = j * T + tid;
             if (FULL || i < nvec) {
                 using Codes = std::conditional_t<ANY, typename IT::codes_any, typename IT::codes>;
-                if constexpr (CPV == 2)
-                    __builtin_nontemporal_store(u32x2{c[j][0], c[j][1]}, reinterpret_cast<Codes *>(dst) + i);
-                else
-                    __builtin_nontemporal_store(c[j][0], reinterpret_cast<Codes *>(dst) + i);
+                Codes q;
+                if constexpr (CPV == 2) q = u32x2{c[j][0], c[j][1]};
+                else q = c[j][0];
+                if constexpr (MODE == ROWS_SHARED) *(reinterpret_cast<Codes *>(dst) + i) = q;
+                else __builtin_nontemporal_store(q, reinterpret_cast<Codes *>(dst) + i);
             }
         }
 
@@ -379,7 +387,7 @@ __global__ __launch_bounds__(256) void row_absmax_kernel(QBatch B, float *__rest
 // weights read once. A wave takes ABSMAX_VPT 16-byte vectors per lane of one row
 // at a time, whatever their alignment (the row's elements past its last whole
 // vector one per lane, with its last piece), the pieces of all rows strided over
-// the waves, so few long rows spread as well as many short ones. bf16 [4099,
+// the waves of as many workgroups as the matrix has rows, 512 at most. bf16 [4099,
 // 4001]: 7.6 us (32.8 MB out of the Infinity Cache) against 54 with 2-byte loads
 // and a barrier per row; 1 or 4 workgroups per CU the same.
 constexpr int ABSMAX_VPT = 8, ABSMAX_WAVES = 8, ABSMAX_BLOCKS_PER_CU = 2, ABSMAX_SLOTS = 512;
@@ -528,6 +536,7 @@ int launch_fast(int key, const QBatch &b, int scheme, float full, hipStream_t st
     case V * 1000 + W * 10 + ROWS_ANY: \
         return launch_fast_t<InT, F, V, W, true, ROWS_ANY>(b, scheme, full, st);
     switch (key) {
+        case 1010 + ROWS_SHARED: return launch_fast_t<InT, F, 1, 1, true, ROWS_SHARED>(b, scheme, full, st);
         RENG_Q(8, 1, 1) RENG_Q(7, 1, 1) RENG_Q(7, 4, 1) RENG_Q(5, 2, 1) RENG_Q(8, 2, 1)
         RENG_Q(8, 4, 1) RENG_Q(6, 9, 1) RENG_Q(2, 1, 1) RENG_Q(4, 1, 1)
         RENG_Q(1, 1, 0) RENG_Q(2, 1, 0) RENG_Q(4, 1, 0) RENG_Q(8, 1, 0) RENG_Q(8, 2, 0)
@@ -583,7 +592,8 @@ int fast_key(const QMat &m, int dtype) {
     const size_t store = dtype == RENG_HIP_BF16 ? 8 : 4;
     const bool aligned = m.cols % epv == 0 && (reinterpret_cast<uintptr_t>(m.w) & 15) == 0 && (m.ld * eb) % 16 == 0 &&
                          (reinterpret_cast<uintptr_t>(m.codes) & (store - 1)) == 0;
-    const FastCfg c = pick_cfg((m.cols + epv - 1) / epv, aligned);
+    FastCfg c = pick_cfg((m.cols + epv - 1) / epv, aligned);
+    if (c.mode == ROWS_ANY && c.vpt == 1 && m.cols % 64 != 0) c.mode = ROWS_SHARED;
     return c.vpt > 0 ? encode_key(c) : -1;
 }
 
