@@ -2,6 +2,9 @@
 // dequantize, the per-row error statistics, and the self-check of the
 // hardware conversion the quantizer's fast path relies on.
 #include "codec.h"
+
+#include <algorithm>
+
 #include "common.h"
 
 namespace reng {
@@ -42,7 +45,8 @@ __global__ void decode_kernel(const uint8_t *__restrict__ c, uint64_t n, float *
 
 // Quantized::dequantize (lib.rs:328-337): decode(code) * scale, one f32
 // multiply; dequantize_bf16 (lib.rs:342-344) rounds that to bf16. Any shape and
-// alignment, one value per thread and step: what dequant_units does not take.
+// alignment, one value per thread and step: small matrices, and what
+// dequant_units does not take (codes or output off a unit's alignment).
 template <int F, bool BF16>
 __global__ void dequant_kernel(const uint8_t *__restrict__ c, const float *__restrict__ scales,
                                uint64_t rows, uint64_t cols, void *__restrict__ out) {
@@ -94,7 +98,7 @@ __device__ __forceinline__ void decode4(uint32_t w, float *v) {
 
 // Bound: HBM (1 byte in, 2 or 4 out per value). The codes are one flat array
 // cut into units of U codes (8 for bf16, 4 for f32 out: one 16-byte store a
-// unit), DQ_UNITS units per thread, requested together, the units of a wave
+// unit), UNITS units per thread, requested together, the units of a wave
 // side by side in each; so any row width divides evenly over the chip. A
 // unit's row comes from its chunk's start (one f64 multiply: the quotient is
 // off by at most one, corrected) plus an f32 division inside the chunk, and a
@@ -104,23 +108,23 @@ __device__ __forceinline__ void decode4(uint32_t w, float *v) {
 // [4096, 14336] to bf16: 95 -> 28 us (a byte load, a 64-bit division and a 2-byte
 // store per value before; 176 MB at the 6.1 TB/s of a mixed stream take 29); 2 or 8
 // units per thread within 2%, 4 workgroups per CU in place of 16 20% slower.
-constexpr int DQ_UNITS = 4, DQ_THREADS = 256;
+constexpr int DQ_THREADS = 256;
 
-template <int F, bool BF16>
+template <int F, bool BF16, int UNITS>
 __global__ __launch_bounds__(DQ_THREADS) void dequant_units(const uint8_t *__restrict__ c,
                                                             const float *__restrict__ scales, uint32_t rows,
                                                             uint64_t cols, double inv_cols, void *__restrict__ out) {
     constexpr int U = BF16 ? 8 : 4;
-    constexpr uint32_t CHUNK = U * DQ_UNITS * DQ_THREADS;   // values per workgroup and step
+    constexpr uint32_t CHUNK = U * UNITS * DQ_THREADS;   // values per workgroup and step
     const uint64_t n = (uint64_t)rows * cols;
     const uint32_t tid = threadIdx.x;
     // Below CHUNK columns a chunk may meet many rows; cols then fits an f32 exactly.
     const bool narrow = cols < CHUNK;
     const float inv32 = narrow ? 1.0f / (float)cols : 0.0f;
     for (uint64_t e0 = (uint64_t)blockIdx.x * CHUNK; e0 < n; e0 += (uint64_t)gridDim.x * CHUNK) {
-        uint32_t q[DQ_UNITS][U / 4];
+        uint32_t q[UNITS][U / 4];
 #pragma unroll
-        for (int j = 0; j < DQ_UNITS; ++j) {
+        for (int j = 0; j < UNITS; ++j) {
             const uint64_t e = e0 + (uint64_t)(j * DQ_THREADS + tid) * U;
             if (e + U <= n) {
                 if constexpr (U == 8) {
@@ -143,7 +147,7 @@ __global__ __launch_bounds__(DQ_THREADS) void dequant_units(const uint8_t *__res
             k0 -= (int64_t)cols;
         }
 #pragma unroll
-        for (int j = 0; j < DQ_UNITS; ++j) {
+        for (int j = 0; j < UNITS; ++j) {
             const uint32_t l = (j * DQ_THREADS + tid) * U;
             const uint64_t e = e0 + l;
             if (e + U > n) continue;
@@ -390,21 +394,34 @@ int launch_decode(const uint8_t *c, uint64_t n, int format, float *out, hipStrea
 
 namespace {
 
+// Four units a thread, or one where four would leave the chip few workgroups (fewer
+// than 4 per CU of 8-code units, 2 of 4-code ones): bf16 [265, 5198] 4.9 -> 3.7 us,
+// [1024, 4096] 6.4 -> 5.3, f32 [1000, 300] 3.9 -> 3.1, while bf16 [4096, 4096] takes
+// 11.8 with one and 10.9 with four, f32 [1024, 4096] 6.4 and 5.5. Below 2^19 values
+// a thread per value is faster still (its chain is shorter: bf16 [2700, 180] 3.0 us
+// against 3.2 with one unit and 5.0 with four; [64, 8192] 3.3 against 3.2).
+constexpr uint64_t DQ_SMALL = 1ull << 19;
+
 template <int F, bool BF16>
 int launch_dequantize_t(const uint8_t *c, const float *scales, uint64_t rows, uint64_t cols, void *out,
                         hipStream_t st) {
-    constexpr uint64_t U = BF16 ? 8 : 4, CHUNK = U * DQ_UNITS * DQ_THREADS;
-    const bool units = cols >= U && rows < (1ull << 31) && rows * cols < (1ull << 52) &&
+    constexpr uint64_t U = BF16 ? 8 : 4, CHUNK = U * DQ_THREADS;
+    const uint64_t n = rows * cols, cus = (uint64_t)device_props().cus;
+    const bool units = n >= DQ_SMALL && cols >= U && rows < (1ull << 31) && n < (1ull << 52) &&
                        (reinterpret_cast<uintptr_t>(c) & (U - 1)) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     if (units) {
-        uint64_t blocks = (rows * cols + CHUNK - 1) / CHUNK;
-        const uint64_t cap = (uint64_t)device_props().cus * 16;
-        if (blocks > cap) blocks = cap;
-        hipLaunchKernelGGL((dequant_units<F, BF16>), dim3((unsigned)blocks), dim3(DQ_THREADS), 0, st, c, scales,
-                           (uint32_t)rows, cols, 1.0 / (double)cols, out);
+        const uint64_t many = BF16 ? 4 : 2;
+        const bool four = n >= many * cus * 4 * CHUNK;
+        const uint64_t chunk = four ? 4 * CHUNK : CHUNK;
+        const dim3 grid((unsigned)std::min((n + chunk - 1) / chunk, cus * 16));
+        if (four)
+            hipLaunchKernelGGL((dequant_units<F, BF16, 4>), grid, dim3(DQ_THREADS), 0, st, c, scales, (uint32_t)rows,
+                               cols, 1.0 / (double)cols, out);
+        else
+            hipLaunchKernelGGL((dequant_units<F, BF16, 1>), grid, dim3(DQ_THREADS), 0, st, c, scales, (uint32_t)rows,
+                               cols, 1.0 / (double)cols, out);
     } else {
-        hipLaunchKernelGGL((dequant_kernel<F, BF16>), stride_grid(rows * cols, 256), dim3(256), 0, st, c, scales, rows,
-                           cols, out);
+        hipLaunchKernelGGL((dequant_kernel<F, BF16>), stride_grid(n, 256), dim3(256), 0, st, c, scales, rows, cols, out);
     }
     return check_launch("dequantize");
 }

@@ -19,6 +19,11 @@ torch = pytest.importorskip("torch")
 
 SHAPES = [(1, 1), (5, 3), (3, 7), (9, 8), (7, 9), (33, 64), (5, 511), (6, 1024), (5, 1031), (3, 8192), (4, 8195),
           (2, 20011), (300, 17), (2100, 40)]
+# Past 2^19 values the expansion runs in units of 8 (bf16) or 4 codes, one a thread, and
+# past 2^23 (2^21 for f32) four: widths of one unit, one value more, no multiple of a
+# unit and wider than a workgroup's chunk.
+UNIT_SHAPES = [(70000, 8), (60000, 9), (1100, 511), (513, 1031), (27, 20011), (1, 600000), (1030000, 9), (65000, 131),
+               (300, 28001)]
 
 
 @pytest.fixture(scope="module")
@@ -44,7 +49,7 @@ def dev(a, shift):
 @pytest.mark.parametrize("shift", [0, 1])
 def test_dequantize_at_unit_edges(R, fmt, shift):
     rng = np.random.default_rng(5)
-    for rows, cols in SHAPES:
+    for rows, cols in SHAPES + UNIT_SHAPES:
         codes = rng.integers(0, 256, rows * cols).astype(np.uint8)
         scales = np.exp2(rng.integers(-20, 20, rows)).astype(np.float32) * np.float32(1.37)
         want = O.Quantized(fmt, "pcs", rows, cols, codes, scales, 0).dequantize()
