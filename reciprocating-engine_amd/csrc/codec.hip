@@ -215,8 +215,7 @@ __global__ __launch_bounds__(DQ_THREADS) void dequant_units(const uint8_t *__res
 // outside 2^-60 .. 2^60 or a reserved code, and rows whose scale passes 2^43, take
 // the IEEE division and the exact decoder. [4096, 14336]: 127 -> 36 us (a 2-byte
 // and a 1-byte load and an IEEE division per weight before; 176 MB take 24.5 us to
-// read). A row per 256-thread workgroup past 1024 weights, below that a wave per
-// row (a workgroup's other waves would have no unit).
+// read). Narrow rows take a weight per lane with the IEEE division (no UNITS).
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 typedef u32x2 u32x2_any __attribute__((aligned(1)));
 
@@ -263,7 +262,7 @@ __device__ __forceinline__ void row_err_unit(const u32x4 &wq, const u32x2 &cq, f
     e.cnt += cnt;
 }
 
-template <int F, int WPR>
+template <int F, int WPR, bool UNITS>
 __global__ __launch_bounds__(256) void row_errors_kernel(const uint16_t *__restrict__ w,
                                                          const uint8_t *__restrict__ c,
                                                          const float *__restrict__ scales,
@@ -285,7 +284,7 @@ __global__ __launch_bounds__(256) void row_errors_kernel(const uint16_t *__restr
             const bool wild = !(__builtin_fabsf(s) <= 0x1p43f);   // |got| may pass 2^59
             const uint16_t *wr = w + r * cols;
             const uint8_t *cr = c + r * cols;
-            const uint64_t units = cols / 8;
+            const uint64_t units = UNITS ? cols / 8 : 0;
             // The next unit is requested before this one's arithmetic (past the
             // row's last unit: that one again).
             u32x4 wn;
@@ -321,7 +320,11 @@ __global__ __launch_bounds__(256) void row_errors_kernel(const uint16_t *__restr
                     row_err_unit<F, true>(wq, cq, s, e);
                 }
             }
-            if (const uint64_t i = units * 8 + t; i < cols) row_err_exact<F>(wr[i], cr[i], s, e);
+            if constexpr (UNITS) {
+                if (const uint64_t i = units * 8 + t; i < cols) row_err_exact<F>(wr[i], cr[i], s, e);
+            } else {
+                for (uint64_t i = t; i < cols; i += T) row_err_exact<F>(wr[i], cr[i], s, e);
+            }
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
@@ -440,18 +443,33 @@ int launch_dequantize(const uint8_t *c, const float *scales, uint64_t rows, uint
 int launch_row_errors(const uint16_t *w, const uint8_t *c, const float *scales, uint64_t cols,
                       uint64_t step, uint64_t nsampled, int format, float *mean_rel,
                       float *max_rel, hipStream_t st) {
-    const bool wave = cols <= 1024;   // two units per lane: a workgroup's other waves would idle
+    const uint64_t cus = (uint64_t)device_props().cus;
+    // A wave per row where a workgroup's other waves would idle and the rows fill the
+    // chip without them; units of eight where a row has enough of them: the IEEE
+    // division of one weight per lane is a shorter chain than a unit and the row's
+    // last weights after it ([244, 12] 4.2 -> 3.4 us, [100, 100] 4.0 -> 3.4, [60000,
+    // 33] 30.7 -> 22.2; the thread-per-weight workgroup that was here first 3.4, 3.4
+    // and 93.3).
+    const bool few = nsampled <= cus;
+    const bool units = cols > 64 && (few ? cols > 256 : cols >= 128);
+    const bool wave = cols <= 64 || (cols <= 1024 && !few);
     uint64_t blocks = wave ? (nsampled + 3) / 4 : nsampled;
-    const uint64_t cap = (uint64_t)device_props().cus * 64;
+    const uint64_t cap = cus * 64;
     if (blocks > cap) blocks = cap;
-#define RENG_ERR(F, WPR)                                                                                             \
-    hipLaunchKernelGGL((row_errors_kernel<F, WPR>), dim3((unsigned)blocks), dim3(256), 0, st, w, c, scales, cols, step, \
-                       nsampled, mean_rel, max_rel)
+#define RENG_ERR(F, WPR, UNITS)                                                                                     \
+    hipLaunchKernelGGL((row_errors_kernel<F, WPR, UNITS>), dim3((unsigned)blocks), dim3(256), 0, st, w, c, scales, cols, \
+                       step, nsampled, mean_rel, max_rel)
+#define RENG_ERR_F(F)                                          \
+    if (wave && units) RENG_ERR(F, 1, true);                   \
+    else if (wave) RENG_ERR(F, 1, false);                      \
+    else if (units) RENG_ERR(F, 4, true);                      \
+    else RENG_ERR(F, 4, false)
     if (format == RENG_HIP_E4M3) {
-        if (wave) RENG_ERR(RENG_HIP_E4M3, 1); else RENG_ERR(RENG_HIP_E4M3, 4);
+        RENG_ERR_F(RENG_HIP_E4M3);
     } else {
-        if (wave) RENG_ERR(RENG_HIP_E5M2, 1); else RENG_ERR(RENG_HIP_E5M2, 4);
+        RENG_ERR_F(RENG_HIP_E5M2);
     }
+#undef RENG_ERR_F
 #undef RENG_ERR
     return check_launch("row_errors");
 }

@@ -24,6 +24,9 @@ SHAPES = [(1, 1), (5, 3), (3, 7), (9, 8), (7, 9), (33, 64), (5, 511), (6, 1024),
 # unit and wider than a workgroup's chunk.
 UNIT_SHAPES = [(70000, 8), (60000, 9), (1100, 511), (513, 1031), (27, 20011), (1, 600000), (1030000, 9), (65000, 131),
                (300, 28001)]
+# The statistics' forms: a weight or a unit of eight per lane, a wave or a workgroup
+# per row, by the width (64, 128, 256, 1024) and by whether the rows pass 256.
+ERR_SHAPES = [(256, 65), (257, 127), (300, 128), (257, 1023), (40, 200), (256, 256), (256, 257), (300, 1031)]
 
 
 @pytest.fixture(scope="module")
@@ -76,7 +79,7 @@ def weights(rng, rows, cols, kind):
 @pytest.mark.parametrize("shift", [0, 1])
 def test_row_errors_at_unit_edges(R, fmt, kind, shift):
     rng = np.random.default_rng(9)
-    for rows, cols in SHAPES:
+    for rows, cols in SHAPES + ERR_SHAPES:
         w = weights(rng, rows, cols, kind)
         ref = O.quantize(w, rows, cols, fmt, "pcs" if kind != "wide" else "unit")
         if kind == "reserved":
