@@ -21,6 +21,7 @@
 #include "common.h"
 #include "gemm.h"
 #include "mfma_pipe.h"
+#include "tile_forms.h"
 
 namespace reng {
 
@@ -36,10 +37,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // What a copy past a row's end reads (TAIL).
 static __device__ const uint32_t zero_chunk[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
 
-// BK codes of k per pipeline stage (64, 128 or 256).
+// BK codes of k per pipeline stage (64 or 128).
 template <int WGM, int WGN, int WM, int WN, int BK>
 struct Tile {
-    static_assert(BK == 64 || BK == 128 || BK == 256, "stage widths");
+    static_assert(BK == 64 || BK == 128, "stage widths");
     static constexpr int W = WGM * WGN;
     static constexpr int BM = 32 * WM * WGM, BN = 32 * WN * WGN;
     static constexpr int A_ROW = 2 * BK, B_ROW = BK;            // bytes of one activation / code row per stage
@@ -53,7 +54,7 @@ struct Tile {
 };
 
 // Chunk slots: chunk c of tile row r sits in slot c ^ swz(r). Activation rows
-// (8-32 chunks) XOR the low three bits of c; code rows use the 4-chunk
+// (8 or 16 chunks) XOR the low three bits of c; code rows use the 4-chunk
 // permutation of mfma_pipe.h for 4 chunks, else the 8-chunk one.
 __device__ __forceinline__ uint32_t swz_a(uint32_t r) { return swz<8>(r); }
 template <int CHB>
@@ -490,65 +491,12 @@ int launch_tiles_cfg(const uint16_t *x, const uint8_t *codes, const float *scale
     return check_launch("w8a16_tiles");
 }
 
-inline uint64_t tile_count(uint32_t M, uint32_t N, uint32_t bm, uint32_t bn) {
-    return (uint64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-}
-
-// Long K (at least 64 stages of 128 codes) over fewer 128 x 128 tiles than
-// half the CUs: one tile per block would leave most of the chip idle.
-inline bool streamk_suits(uint32_t M, uint32_t N, uint32_t K) {
-    return K % 128 == 0 && K >= 8192 && 2 * tile_count(M, N, 128, 128) < (uint64_t)device_props().cus;
-}
-
-// Tile choice. Long K (K >= 8192) over fewer 128 x 128 tiles than half the
-// CUs runs stream-K on 128 x 128 tiles of 128-code stages (M = 256
-// [4096, 14336]: 92.8 -> 66.5 us). Otherwise each form's time is modelled as
-// rounds x (c0 + c1 x K / 64), rounds = ceil(tiles / CUs), with (c0, c1) in
-// microseconds fitted to graph-replayed timings of every form on eleven
-// products (M 128-1024 over the Llama-3.1-8B and Qwen2.5-32B shapes; most
-// within 16% of the fit), scaled per form to this pipeline's times (0.91-0.93;
-// 256 x 256 and 64 x 64 1.06-1.08), and the cheapest form runs. On 22 products
-// (M 80-1024, N 1200-28672, K 1024-10240) the picks were all faster than
-// those of the earlier fit and pipeline, by 4-33% (M = 700 [3000, 2048] 25.5
-// -> 17.3 us, M = 150 [25000, 1536] 31.0 -> 23.4). Stream-K takes
-// (G + tiles - 1) BM BN floats of partials (6.3 Mi floats at most on 256
-// CUs) and a counter per tile (fewer than 128).
-struct TilePick {
-    int form;
-    float est;   // modelled microseconds
-};
-
-inline TilePick tile_pick(uint32_t M, uint32_t N, uint32_t K) {
-    struct Cand {
-        uint32_t bm, bn;
-        float c0, c1;
-        bool fits;
-    };
-    const Cand cands[] = {
-        {256, 256, 28.6f, 1.200f, true},                            // 8 waves of 128 x 64, 64-code stages, 3 slots
-        {128, 256, 16.6f, 0.650f, true},                            // 8 waves of 64 x 64
-        {128, 160, 5.2f, 0.650f, K % 64 != 0 || K % 128 == 0},      // 4 waves of 32 x 160, 128-code stages, 2 slots
-        {128, 128, 9.3f, 0.425f, true},                             // 8 waves of 64 x 32, 64-code stages, 6 slots
-        {64, 128, 4.6f, 0.318f, true},                              // 8 waves of 32 x 32
-        {64, 64, 0.0f, 0.270f, true},                               // 4 waves of 32 x 32
-    };
-    const uint64_t cus = (uint64_t)device_props().cus;
-    TilePick best{0, 0.0f};
-    for (int i = 0; i < 6; ++i) {
-        if (!cands[i].fits) continue;
-        const uint64_t rounds = (tile_count(M, N, cands[i].bm, cands[i].bn) + cus - 1) / cus;
-        const float est = (float)rounds * (cands[i].c0 + cands[i].c1 * (float)((K + 63) / 64));
-        if (i == 0 || est < best.est) best = TilePick{i, est};
-    }
-    return best;
-}
-
 template <int F>
 int launch_tiles_f(const uint16_t *x, const uint8_t *codes, const float *scales, uint32_t M, uint32_t N,
                    uint32_t K, uint16_t *y, hipStream_t st, const SplitScratch *fixed) {
     const uint64_t cus = (uint64_t)device_props().cus;
     const uint64_t t128 = tile_count(M, N, 128, 128);
-    if (streamk_suits(M, N, K)) {
+    if (streamk_suits(M, N, K, cus)) {
         using T = Tile<2, 4, 2, 1, 128>;
         const uint64_t units = t128 * (K / 128);
         const uint32_t grid = (uint32_t)(units < cus ? units : cus);
@@ -574,12 +522,12 @@ int launch_tiles_f(const uint16_t *x, const uint8_t *codes, const float *scales,
     const bool wide = K % 128 == 0;
 #define RENG_TILES_128(...)                                                                                      \
     return launch_tiles_cfg<F, __VA_ARGS__, false>(x, codes, scales, M, N, K, y, st, 0, nullptr, nullptr)
-    switch (tile_pick(M, N, K).form) {
-    case 0: RENG_TILES(2, 4, 4, 2, 64, 3);
-    case 1: if (wide) RENG_TILES_128(2, 4, 2, 2, 128, 2); RENG_TILES(2, 4, 2, 2, 64, 3);
-    case 2: RENG_TILES(4, 1, 1, 5, 128, 2);
-    case 3: RENG_TILES(2, 4, 2, 1, 64, 6);
-    case 4: if (wide) RENG_TILES_128(2, 4, 1, 1, 128, 4); RENG_TILES(2, 4, 1, 1, 64, 6);
+    switch (tile_pick(M, N, K, cus).form) {
+    case TILES_256x256: RENG_TILES(2, 4, 4, 2, 64, 3);
+    case TILES_128x256: if (wide) RENG_TILES_128(2, 4, 2, 2, 128, 2); RENG_TILES(2, 4, 2, 2, 64, 3);
+    case TILES_128x160: RENG_TILES(4, 1, 1, 5, 128, 2);
+    case TILES_128x128: RENG_TILES(2, 4, 2, 1, 64, 6);
+    case TILES_64x128: if (wide) RENG_TILES_128(2, 4, 1, 1, 128, 4); RENG_TILES(2, 4, 1, 1, 64, 6);
     default: if (wide) RENG_TILES_128(2, 2, 1, 1, 128, 3); RENG_TILES(2, 2, 1, 1, 64, 6);
     }
 #undef RENG_TILES_128
@@ -588,23 +536,8 @@ int launch_tiles_f(const uint16_t *x, const uint8_t *codes, const float *scales,
 
 }  // namespace tiles
 
-// K % 64 == 0: below half the CUs in 64 x 128 tiles the 64-row kernels, which
-// split K, are faster (M = 100 [3000, 4096]: 22.2 against 28.1 us) - unless
-// the product suits stream-K. K no multiple of 128: the 64-row launches, each
-// about 6 us + N K / 2.9 TB/s there (M = 128 [14336, 4112] 25 us a launch,
-// M = 300 [3000, 3600] 10, M = 700 [1500, 1296] 7.4), against the tiles' own
-// model, a quarter added for the short stage's checks and few tiles (M = 70
-// [4000, 6160]: tiles 30.8 us, two launches 27.7). M = 256 [4096, 4112] 54.1 ->
-// 22.7 us, M = 300 [3000, 3600] 50.2 -> 20.7, M = 1000 [10000, 1552] 174 -> 51,
-// M = 1024 [2048, 16400] 340 -> 105.
 bool w8a16_tiles_take(uint32_t M, uint32_t N, uint32_t K) {
-    if (M <= 64) return false;
-    if (K % 64 == 0 &&
-        (tiles::streamk_suits(M, N, K) || 2 * tiles::tile_count(M, N, 64, 128) >= (uint64_t)device_props().cus))
-        return true;
-    if (K % 128 == 0) return false;
-    const float loop = (float)((M + 63) / 64) * (6.0f + (float)N * (float)K / 2.9e6f);
-    return 1.25f * tiles::tile_pick(M, N, K).est < loop;
+    return tiles::tiles_take(M, N, K, (uint64_t)device_props().cus);
 }
 
 int launch_w8a16_tiles(const uint16_t *x, const uint8_t *codes, const float *scales, uint32_t M, uint32_t N,

@@ -63,3 +63,21 @@ def test_fp8_test_shapes_run_every_wide_form():
     wide = {f for f in D.FP8_FORMS if f.startswith("wide")}
     assert {c[3] for c in G.FP8_WIDE} == wide
     assert {c[3] for c in G.FP8_RAGGED} & wide == wide - {"wide 64x64"}
+
+
+@pytest.mark.parametrize("M,N,K,fmt,form", G.W8A16_TILES + G.W8A16_STAGES_128 + G.W8A16_TAIL)
+def test_w8a16_test_shapes_run_the_forms_they_name(M, N, K, fmt, form):
+    assert D.w8a16_form(M, N, K) == form
+
+
+def test_w8a16_test_shapes_run_every_form():
+    """All six tiles whole and with a short last stage, and, of the three that
+    have two stage widths, both."""
+    six = set(D.W8A16_FORMS[:6])
+    assert {c[4] for c in G.W8A16_TILES} == six and {c[4] for c in G.W8A16_TAIL} == six
+    assert all(c[2] % 64 == 0 for c in G.W8A16_TILES) and all(c[2] % 64 for c in G.W8A16_TAIL)
+    two = {"128x256", "64x128", "64x64"}
+    assert {c[4] for c in G.W8A16_STAGES_128} == two and all(c[2] % 128 == 0 for c in G.W8A16_STAGES_128)
+    assert two <= {c[4] for c in G.W8A16_TILES if c[2] % 128}
+    assert D.w8a16_form(256, 2048, 8192) == D.w8a16_form(200, 1000, 8320) == "stream-K"
+    assert D.w8a16_form(100, 3000, 4096) == "64 rows"

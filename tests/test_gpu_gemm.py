@@ -422,43 +422,61 @@ def test_skinny_every_output_of_a_qwen_7b_gate_up(R, M):
     check_w8a16(R, rng, M, 18944, 3584, E4M3)
 
 
-@pytest.mark.parametrize("M, N, K, fmt", [
-    (1000, 12288, 1024, E4M3),  # 256 x 256 tiles; ragged M
-    (384, 20480, 1024, E5M2),   # 128 x 256 tiles
-    (200, 20480, 768, E4M3),    # 128 x 160 tiles (4 waves, 128-code stages); ragged M
-    (200, 20001, 768, E5M2),    # 128 x 160 tiles; ragged M and N (element stores)
-    (768, 4097, 1536, E5M2),    # 128 x 128 tiles; ragged N (element stores)
-    (200, 4097, 3072, E4M3),    # 64 x 128 tiles; ragged M and N
-    (96, 8192, 64, E5M2),       # 64 x 64 tiles (4 waves); one stage
-    (512, 8192, 192, E4M3),     # 64 x 64 tiles; K % 128 != 0
-])
+# The form the launcher's cost model picks on a 256-CU MI355X beside each shape.
+W8A16_TILES = [
+    (711, 20554, 640, E4M3, "256x256"),     # ragged M and N (element stores)
+    (384, 20480, 1024, E5M2, "128x256"),
+    (328, 19168, 704, E4M3, "128x256"),     # 64-code stages; ragged M and N
+    (1000, 12288, 1024, E4M3, "128x160"),   # ragged M and N
+    (200, 20480, 768, E4M3, "128x160"),     # 4 waves, 128-code stages; ragged M
+    (200, 20001, 768, E5M2, "128x160"),     # ragged M and N (element stores)
+    (768, 4097, 1536, E5M2, "128x128"),     # ragged N (element stores)
+    (200, 4097, 3072, E4M3, "64x128"),      # ragged M and N
+    (66, 8263, 1344, E5M2, "64x128"),       # 64-code stages
+    (96, 8192, 64, E5M2, "64x64"),          # 4 waves; one stage
+    (512, 8192, 192, E4M3, "64x64"),        # K % 128 != 0
+]
+
+
+@pytest.mark.parametrize("M, N, K, fmt", [c[:4] for c in W8A16_TILES])
 def test_w8a16_tiles_every_output(R, M, N, K, fmt):
-    """More than 64 activation rows take the tiled bf16-MFMA kernel; one shape
-    per tile form the launcher's cost model picks on a 256-CU MI355X, every
-    output against the oracle and float64."""
+    """More than 64 activation rows take the tiled bf16-MFMA kernel: every tile
+    form the launcher picks, every output against the oracle and float64."""
     rng = np.random.default_rng(M * 7 + N + K)
     check_w8a16(R, rng, M, N, K, fmt)
 
 
-@pytest.mark.parametrize("M, N, K, fmt", [
-    (520, 16300, 256, E4M3),    # 128 x 256 tiles over two stages, ragged M and N
-    (200, 4097, 1152, E5M2),    # 64 x 128 tiles, more stages than slots
-    (130, 8190, 128, E4M3),     # one stage
-    (96, 8200, 384, E5M2),      # 64 x 64 tiles, as many stages as slots
-])
+W8A16_STAGES_128 = [
+    (129, 27941, 1152, E4M3, "128x256"),    # nine stages over two slots, ragged M and N
+    (65, 8811, 1408, E5M2, "64x128"),       # more stages than slots, ragged M and N
+    (200, 4097, 1152, E5M2, "64x64"),       # more stages than slots
+    (520, 16300, 256, E4M3, "64x64"),       # two stages, ragged M and N
+    (130, 8190, 128, E4M3, "64x64"),        # one stage
+    (96, 8200, 384, E5M2, "64x64"),         # as many stages as slots
+]
+
+
+@pytest.mark.parametrize("M, N, K, fmt", [c[:4] for c in W8A16_STAGES_128])
 def test_w8a16_tiles_of_128_code_stages(R, M, N, K, fmt):
     """K a multiple of 128: the narrower tile forms stage 128 codes at a time."""
     check_w8a16(R, np.random.default_rng(M * 3 + N + K), M, N, K, fmt)
 
 
-@pytest.mark.parametrize("M, N, K, fmt", [
-    (1024, 16390, 80, E4M3),    # 256 x 256 tiles; a short second stage
-    (520, 16300, 144, E5M2),    # 128 x 256 tiles; one chunk in the last stage
-    (1000, 5100, 176, E4M3),    # 128 x 160 tiles; 48 codes past a whole stage
-    (768, 4097, 1552, E5M2),    # 128 x 128 tiles; ragged N
-    (200, 4097, 3120, E4M3),    # 64 x 128 tiles
-    (96, 8192, 16, E5M2),       # 64 x 64 tiles; one chunk in all
-])
+W8A16_TAIL = [
+    (705, 20501, 608, E5M2, "256x256"),     # 32 codes past a whole stage; ragged M and N
+    (326, 19352, 656, E4M3, "128x256"),     # one chunk in the last stage
+    (68, 25265, 784, E5M2, "128x160"),      # 128-code stages, one chunk in the last; element stores
+    (200, 17048, 560, E4M3, "128x160"),     # 48 codes past a whole stage
+    (768, 4097, 1552, E5M2, "128x128"),     # ragged N
+    (200, 4097, 3120, E4M3, "64x128"),
+    (96, 8192, 16, E5M2, "64x64"),          # one chunk in all
+    (1024, 16390, 80, E4M3, "64x64"),       # a short second stage
+    (520, 16300, 144, E5M2, "64x64"),       # one chunk in the last stage
+    (1000, 5100, 176, E4M3, "64x64"),       # 48 codes past a whole stage
+]
+
+
+@pytest.mark.parametrize("M, N, K, fmt", [c[:4] for c in W8A16_TAIL])
 def test_w8a16_tiles_short_last_stage(R, M, N, K, fmt):
     """More than 64 activation rows and K a multiple of 16 but not of 64: the
     tiled kernel's last stage is padded with zeros. x and the codes are views
