@@ -478,7 +478,8 @@ def _attention_want(Q, K, V, nh, nkv, hd, scale):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("nh,nkv,hd", [(6, 2, 64), (32, 8, 128), (4, 4, 6), (2, 1, 1024), (16, 1, 128)])
+@pytest.mark.parametrize("nh,nkv,hd", [(6, 2, 64), (32, 8, 128), (4, 4, 6), (2, 1, 1024), (16, 1, 128), (8, 2, 96),
+                                       (16, 4, 96), (16, 4, 32)])
 def test_attention_forms_against_numpy(nh, nkv, hd):
     """Both attention entry points against float64 numpy softmax attention:
     lengths around the 256-row tile and the one-pass limit (512 rows), caches
