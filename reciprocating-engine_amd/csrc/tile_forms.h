@@ -29,7 +29,11 @@ inline bool streamk_suits(uint32_t M, uint32_t N, uint32_t K, uint64_t cus) {
 // 256 x 256 and 64 x 64 1.06-1.08), and the cheapest form runs. On 22 products
 // (M 80-1024, N 1200-28672, K 1024-10240) the picks were all faster than
 // those of the earlier fit and pipeline, by 4-33% (M = 700 [3000, 2048] 25.5
-// -> 17.3 us, M = 150 [25000, 1536] 31.0 -> 23.4). Stream-K takes
+// -> 17.3 us, M = 150 [25000, 1536] 31.0 -> 23.4). The constants of 128 x 256,
+// 64 x 128 and 64 x 64 are those of 128-code stages; K = 64 mod 128 and the padded K
+// run 64-code ones on them, and their picks are within 2 and 3% of the fastest form
+// (70 random products each, the worst 22 and 26%; none slower than before the refit,
+// the first kind 36% faster in the mean). Stream-K takes
 // (G + tiles - 1) BM BN floats of partials (6.3 Mi floats at most on 256
 // CUs) and a counter per tile (fewer than 128).
 enum TileForm { TILES_256x256, TILES_128x256, TILES_128x160, TILES_128x128, TILES_64x128, TILES_64x64 };
