@@ -485,9 +485,10 @@ def test_attention_forms_against_numpy(nh, nkv, hd):
     lengths around the 256-row tile and the one-pass limit (512 rows), caches
     that take several tiles per split and 64 splits, head_dim not a multiple
     of 8 (the 4-byte key path), head_dim 1024, one key/value head for 16 query
-    heads, and a key cache 4 bytes off a 16-byte boundary (the 4-byte key path
-    at head_dim % 8 == 0). The split form's workspace starts as NaN, so a split
-    it fails to write shows up."""
+    heads, head_dim 96 and 32 (the general 16-byte kernel: 20000 rows are 64
+    splits, two heads a workgroup of 8 heads and four of 16), and a key cache 4
+    bytes off a 16-byte boundary (the 4-byte key path at head_dim % 8 == 0). The
+    split form's workspace starts as NaN, so a split it fails to write shows up."""
     import torch
 
     import reng_hip as R
