@@ -273,20 +273,23 @@ RENG_HIP_API int reng_hip_rope_append(uint16_t *q, const uint16_t *k, const uint
 /* One query per head over cache rows 0 .. len - 1 (layer_cpu's causal attention,
  * model.rs:3010-3050): out[h] = softmax(scale * q[h] . K[:, g]) V[:, g] with
  * g = h / (n_heads / n_kv_heads), bf16 in and out, f32 inside (online softmax
- * over tiles of rows); 1 <= len <= RENG_HIP_ATTENTION_MAX_LEN; q, k_cache
- * and v_cache 4-byte aligned. One workgroup per query head reads the whole
- * cache: for longer caches use reng_hip_attention_decode_split. */
+ * over tiles of rows; a NaN score makes its head's output NaN); 1 <= len <= RENG_HIP_ATTENTION_MAX_LEN; q, k_cache and
+ * v_cache 4-byte aligned. One pass: a workgroup per query head (or group of up
+ * to four that share a key/value head, for 64 and 128 dimensions) reads the
+ * whole cache, so for longer caches use reng_hip_attention_decode_split. */
 RENG_HIP_API int reng_hip_attention_decode(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v_cache,
                                            size_t n_heads, size_t n_kv_heads, size_t head_dim, size_t len,
                                            float scale, uint16_t *out, void *stream);
 
-/* Bytes of device workspace reng_hip_attention_decode_split needs for every
- * cache length from 1 to len (0 when all of them take one pass: len <= 512). */
+/* Bytes of device workspace reng_hip_attention_decode_split asks for, for every
+ * cache length from 1 to len (0 for len <= 512). */
 RENG_HIP_API size_t reng_hip_attention_workspace_bytes(size_t n_heads, size_t head_dim, size_t len);
 
-/* reng_hip_attention_decode that, past 512 cache rows, cuts the cache into
- * min(64, ceil(len / 256)) splits, one workgroup per split and group of query
- * heads sharing a key/value head (each split's rows read once for the group);
+/* reng_hip_attention_decode that cuts longer caches into min(64, ceil(len / 256))
+ * splits: past 1024 rows for heads of 64 and 128 dimensions over 16-byte
+ * aligned q and caches (splits of whole 64-row tiles, up to sixteen query heads
+ * a workgroup), else past 512 (up to four heads a workgroup). A workgroup takes
+ * a split and a group of query heads that share a key/value head;
  * the splits' unnormalised outputs and softmax statistics go to workspace
  * (f32, 4-byte aligned, workspace_bytes >= reng_hip_attention_workspace_bytes(
  * n_heads, head_dim, len)) and a second kernel merges them. Asynchronous on
