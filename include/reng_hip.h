@@ -273,10 +273,11 @@ RENG_HIP_API int reng_hip_rope_append(uint16_t *q, const uint16_t *k, const uint
 /* One query per head over cache rows 0 .. len - 1 (layer_cpu's causal attention,
  * model.rs:3010-3050): out[h] = softmax(scale * q[h] . K[:, g]) V[:, g] with
  * g = h / (n_heads / n_kv_heads), bf16 in and out, f32 inside (online softmax
- * over tiles of rows; a NaN score makes its head's output NaN); 1 <= len <= RENG_HIP_ATTENTION_MAX_LEN; q, k_cache and
- * v_cache 4-byte aligned. One pass: a workgroup per query head (or group of up
- * to four that share a key/value head, for 64 and 128 dimensions) reads the
- * whole cache, so for longer caches use reng_hip_attention_decode_split. */
+ * over tiles of rows; a NaN score makes its head's output NaN);
+ * 1 <= len <= RENG_HIP_ATTENTION_MAX_LEN; q, k_cache and v_cache 4-byte
+ * aligned. One pass: a workgroup per query head (or group of up to four that
+ * share a key/value head, for 64 and 128 dimensions) reads the whole cache, so
+ * for longer caches use reng_hip_attention_decode_split. */
 RENG_HIP_API int reng_hip_attention_decode(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v_cache,
                                            size_t n_heads, size_t n_kv_heads, size_t head_dim, size_t len,
                                            float scale, uint16_t *out, void *stream);

@@ -523,10 +523,11 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_split16(
 // waves side by side take the same rows for as many groups of heads, so that
 // the rows come from HBM once and from L2 after that.
 //
-// One call, 32 heads on 8 of 128 dimensions, attention_split16 before: 64 rows
-// 5.9 -> 4.0 us, 512 rows 8.6 -> 6.0, 4096 rows 14.8 -> 12.0, 32768 rows 47.3
-// -> 31.8 (the rows at 4.9 TB/s, then the merge); 28 heads on 4, 32768 rows:
-// 88.8 -> 24.2; 40 on 8: 121 -> 38.
+// One call, 32 heads on 8 of 128 dimensions, attention_split16 before, caches in
+// turn past the Infinity Cache: 64 rows 6.0 -> 4.1 us, 512 rows 8.6 -> 6.1, 4096
+// rows 14.8 -> 12.0, 32768 rows 53.2 -> 39.1 (the rows in 33.5 us, 4.0 TB/s, each
+// read once from HBM, then the merge); 20000 rows, 28 heads on 4: 71 -> 21, 40 on
+// 8: 104 -> 33, 8 on 2: 18.0 -> 13.4.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
