@@ -234,7 +234,10 @@ __global__ __launch_bounds__(64 * WAVES) void quantize_rows_fast(QBatch B, int s
         if constexpr (CLAMP) {
             if (scheme == RENG_HIP_HW && mi != hw_mi) {
                 hw_mi = mi;
-                hw_s = M.scales[0];   // hw_bias_kernel's, for every row of the matrix
+                // hw_bias_kernel's, for every row of the matrix; in a scalar register (in a
+                // vector one it cost the 16-wave form, which spills, 8-16%: bf16 [2000,
+                // 40960] unit 51 -> 59 us).
+                hw_s = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(M.scales[0])));
             }
             s = scheme == RENG_HIP_PCS ? pcs_scale<InT>(mx, full) : hw_s;
         } else {
