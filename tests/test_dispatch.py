@@ -81,3 +81,15 @@ def test_w8a16_test_shapes_run_every_form():
     assert two <= {c[4] for c in G.W8A16_TILES if c[2] % 128}
     assert D.w8a16_form(256, 2048, 8192) == D.w8a16_form(200, 1000, 8320) == "stream-K"
     assert D.w8a16_form(100, 3000, 4096) == "64 rows"
+
+
+@pytest.mark.parametrize("M,N,K,form", [
+    # Short K over many rounds, which a model fitted on long K priced too low.
+    (780, 26741, 640, "128x256"), (895, 13283, 1024, "256x256"), (166, 19625, 4080, "128x160"),
+    # The sizes in use, and few tiles over a K that no whole stage divides.
+    (256, 4096, 4096, "64x64"), (256, 14336, 4096, "128x128"), (512, 5120, 5120, "128x128"),
+    (1024, 5120, 5120, "128x160"), (1024, 27648, 5120, "256x256"), (1024, 5120, 27648, "128x160"),
+    (256, 4096, 14336, "stream-K"), (86, 5636, 16944, "64 rows"), (70, 4000, 6160, "64 rows"),
+])
+def test_w8a16_forms(M, N, K, form):
+    assert D.w8a16_form(M, N, K) == form

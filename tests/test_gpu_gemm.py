@@ -427,14 +427,16 @@ W8A16_TILES = [
     (711, 20554, 640, E4M3, "256x256"),     # ragged M and N (element stores)
     (384, 20480, 1024, E5M2, "128x256"),
     (328, 19168, 704, E4M3, "128x256"),     # 64-code stages; ragged M and N
-    (1000, 12288, 1024, E4M3, "128x160"),   # ragged M and N
-    (200, 20480, 768, E4M3, "128x160"),     # 4 waves, 128-code stages; ragged M
-    (200, 20001, 768, E5M2, "128x160"),     # ragged M and N (element stores)
+    (1000, 12288, 1024, E4M3, "256x256"),   # ragged M
+    (200, 20480, 768, E4M3, "128x256"),     # ragged M
+    (200, 20001, 768, E5M2, "128x256"),     # ragged M and N (element stores)
+    (193, 16648, 896, E4M3, "128x160"),     # 4 waves, 128-code stages; ragged M and N
+    (193, 16645, 896, E5M2, "128x160"),     # element stores
     (768, 4097, 1536, E5M2, "128x128"),     # ragged N (element stores)
     (200, 4097, 3072, E4M3, "64x128"),      # ragged M and N
     (66, 8263, 1344, E5M2, "64x128"),       # 64-code stages
     (96, 8192, 64, E5M2, "64x64"),          # 4 waves; one stage
-    (512, 8192, 192, E4M3, "64x64"),        # K % 128 != 0
+    (512, 8192, 192, E4M3, "128x128"),      # K % 128 != 0
 ]
 
 
@@ -449,8 +451,9 @@ def test_w8a16_tiles_every_output(R, M, N, K, fmt):
 W8A16_STAGES_128 = [
     (129, 27941, 1152, E4M3, "128x256"),    # nine stages over two slots, ragged M and N
     (65, 8811, 1408, E5M2, "64x128"),       # more stages than slots, ragged M and N
-    (200, 4097, 1152, E5M2, "64x64"),       # more stages than slots
-    (520, 16300, 256, E4M3, "64x64"),       # two stages, ragged M and N
+    (200, 4097, 1152, E5M2, "64x128"),
+    (250, 4090, 1024, E5M2, "64x64"),       # more stages than slots, ragged M and N
+    (200, 4097, 256, E4M3, "64x64"),        # two stages
     (130, 8190, 128, E4M3, "64x64"),        # one stage
     (96, 8200, 384, E5M2, "64x64"),         # as many stages as slots
 ]
@@ -465,14 +468,16 @@ def test_w8a16_tiles_of_128_code_stages(R, M, N, K, fmt):
 W8A16_TAIL = [
     (705, 20501, 608, E5M2, "256x256"),     # 32 codes past a whole stage; ragged M and N
     (326, 19352, 656, E4M3, "128x256"),     # one chunk in the last stage
-    (68, 25265, 784, E5M2, "128x160"),      # 128-code stages, one chunk in the last; element stores
+    (222, 16493, 400, E5M2, "128x160"),     # 128-code stages, one chunk in the last; element stores
     (200, 17048, 560, E4M3, "128x160"),     # 48 codes past a whole stage
     (768, 4097, 1552, E5M2, "128x128"),     # ragged N
+    (68, 25265, 784, E5M2, "128x128"),      # one chunk in the last stage; element stores
     (200, 4097, 3120, E4M3, "64x128"),
     (96, 8192, 16, E5M2, "64x64"),          # one chunk in all
-    (1024, 16390, 80, E4M3, "64x64"),       # a short second stage
-    (520, 16300, 144, E5M2, "64x64"),       # one chunk in the last stage
-    (1000, 5100, 176, E4M3, "64x64"),       # 48 codes past a whole stage
+    (250, 4000, 176, E4M3, "64x64"),        # 48 codes past a whole stage
+    (1024, 16390, 80, E4M3, "128x256"),     # a short second stage
+    (520, 16300, 144, E5M2, "128x128"),     # one chunk in the last stage
+    (1000, 5100, 176, E4M3, "128x256"),     # 48 codes past a whole stage
 ]
 
 
