@@ -39,7 +39,7 @@ def test_attention_stream_plan(nh, nkv):
 
 
 @pytest.mark.parametrize("M,N,K,form", [
-    # The clamped-row kernel where no wide tile divides the product and it is ahead: two 128 x 128
+    # The clamped-row kernel where it is ahead of the wide forms: two 128 x 128
     # workgroups on a CU, and 256 x 128 for short M over long K.
     (271, 19624, 3328, "rows 128x128"), (560, 11144, 4864, "rows 128x128"), (324, 20696, 3968, "rows 128x128"),
     (136, 25912, 10752, "rows 256x128"),

@@ -615,13 +615,14 @@ def test_fp8_gemm_wide_tiles(R, M, N, K, fa, fb):
 
 
 # M and N that no tile divides, over every wide form but 64 x 64: tiles past the
-# edge move back onto their neighbour's outputs. Where 64 x 64 tiles or a form of
-# the clamped-row kernel are the cheapest, that kernel runs ("rows"), down to one
-# row or column past a tile.
+# edge move back onto their neighbour's outputs. Where 64 x 64 tiles or a larger
+# form of the clamped-row kernel are the cheapest, that kernel runs ("rows"), down
+# to one row or column past a tile.
 FP8_RAGGED = [(1000, 16376, 256, "wide 256x256"), (330, 13800, 1152, "wide 256x128"), (1000, 4104, 1024, "wide 128x160"),
-              (1000, 5112, 1024, "wide 128x160"), (203, 13008, 1024, "wide 128x128"), (1000, 27640, 256, "wide mixed"),
+              (1000, 5112, 1024, "wide 128x160"), (203, 13008, 1024, "wide 128x128"), (1000, 25080, 2048, "wide mixed"),
               (64, 72, 128, "rows 64x64"), (65, 64, 256, "rows 64x64"), (127, 1000, 384, "rows 64x64"),
-              (333, 4104, 640, "rows 64x64"), (520, 16392, 384, "rows 128x128"), (262, 11288, 1024, "rows 128x128")]
+              (333, 4104, 640, "rows 64x64"), (520, 16392, 384, "wide 256x256"), (262, 11288, 1024, "wide 128x160"),
+              (262, 16392, 256, "rows 128x128"), (520, 11144, 1024, "rows 128x128")]
 
 
 @pytest.mark.parametrize("M,N,K", [c[:3] for c in FP8_RAGGED])
